@@ -59,6 +59,25 @@ def test_quantize_is_the_oracle(bits, g, dtype, n, k):
     np.testing.assert_array_equal(torch_to_act(b, dtype), ob)
 
 
+@pytest.mark.parametrize("bits,g,dtype,n,k", [(4, 32, "f16", 1, 32), (8, 128, "bf16", 3, 128),
+                                              (4, 64, "bf16", 5, 448), (8, 32, "f16", 7, 96)])
+def test_quantize_ties_and_unaligned_weights(bits, g, dtype, n, k):
+    """Values on a coarse grid put quotients exactly between codes; a view one element into its
+    storage is only 2-byte aligned. Codes, scales and biases are the oracle's bit for bit."""
+    rng = np.random.default_rng(n * 11 + k + bits)
+    w = O.from_f32((np.rint(rng.standard_normal((n, k)) * 6) * 0.125).astype(np.float32), dtype)
+    ow, os_, ob = O.affine_quantize(w, g, bits, dtype)
+    aligned = act_to_torch(w, dtype)
+    store = torch.empty(n * k + 1, dtype=aligned.dtype, device=aligned.device)
+    shifted = store[1:].view(n, k)
+    shifted.copy_(aligned)
+    for weight in (aligned, shifted):
+        w_q, s, b = mt.affine_quantize(weight, group_size=g, bits=bits)
+        np.testing.assert_array_equal(w_q.cpu().numpy().view(np.uint32), ow)
+        np.testing.assert_array_equal(torch_to_act(s, dtype), os_)
+        np.testing.assert_array_equal(torch_to_act(b, dtype), ob)
+
+
 def test_compressed_down_weight_projects_like_the_oracle():
     rng = np.random.default_rng(5)
     dense = O.from_f32((rng.standard_normal((1536, 1024)) * 0.02).astype(np.float32), "bf16")
