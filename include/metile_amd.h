@@ -73,6 +73,16 @@ int mt_affine_swiglu(const void* x, const uint32_t* gate_w, const void* gate_sca
 /* Workspace bytes for mt_affine_mlp (hidden activation plus split-K partials). */
 size_t mt_affine_mlp_workspace_bytes(int M, int H, int I, int group_size, int bits);
 
+/* Calls of more rows than one small-row dispatch takes (32; 16 for groups of 32) run as one launch
+ * of the wide kernel, which reads the weights once per row tile of up to 128 rows, where the format
+ * allows (4-bit groups of 64 or more, 8-bit groups of 32 or more; x and y below 2 GiB) and the
+ * workspace holds its split-K partials: at least these many bytes. With less they run as row
+ * dispatches within the sizes of the queries above. The first is what the wide kernel needs (0 where
+ * it does not apply or does not split K), the second at least mt_affine_mlp_workspace_bytes. No
+ * counterpart in the reference, whose row kernels loop. */
+size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int bits, int nproj);
+size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits);
+
 /* y = down(swiglu(x)) (+ residual), x [M, H], gate/up [I, H], down [H, I]. The hidden
  * activation is rounded to the activation dtype between the two kernels, as the reference
  * executor's two dispatches do. Replaces the execute() closure of mlx_affine_mlp_executor
@@ -174,8 +184,10 @@ size_t mt_affine_gemm_workspace_bytes(int M, int K, int N, int group_size, int b
 
 /* y = x @ dequantize(w_q)^T for many rows (prefill) on the matrix cores with fp32 accumulation.
  * Dequantization stays exact: the codes enter the MFMAs as exact 16-bit floats (offset + q) and
- * each 64-wide step's partial gets its group's scale and bias terms in fp32. Replaces mlx_affine_matmul / lower_affine_matmul
- * (metile/backends/mlx_affine.py:359-406, metile/compiler/affine_quantized.py:7-99).
+ * each 64-wide step's partial gets its group's scale and bias terms in fp32. More than 32 rows with
+ * no plan installed for the shape take the wide kernel, given its workspace
+ * (mt_affine_rows_workspace_bytes); otherwise the installed or the planner's plan below runs.
+ * Replaces mlx_affine_matmul / lower_affine_matmul (metile/backends/mlx_affine.py:359-406, metile/compiler/affine_quantized.py:7-99).
  * bits = 4; group_size a power of two >= 64 dividing K; K % 64 == 0; N % 32 == 0. */
 int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const void* biases,
                    void* y, int M, int K, int N, int group_size, int bits, int dtype,
@@ -289,7 +301,8 @@ int mt_affine_qmv_plan_candidates(int M, int K, int N, int group_size, int bits,
 /* Install `plan` for the shape (rejects a plan the kernels cannot run); NULL removes it. */
 int mt_affine_qmv_plan_set(int M, int K, int N, int group_size, int bits, int nproj, int dtype,
                            const mt_qmv_plan* plan);
-/* The same three for the prefill GEMM (4-bit; M = rows of the call, bucketed likewise). */
+/* The same three for the prefill GEMM (4-bit; M = rows of the call, bucketed likewise). With no plan
+ * installed the first gives the planner's, which runs where the wide kernel does not. */
 int mt_affine_gemm_plan(int M, int K, int N, int group_size, int dtype, mt_gemm_plan* out);
 int mt_affine_gemm_plan_candidates(int M, int K, int N, int group_size, mt_gemm_plan* out,
                                    int capacity);

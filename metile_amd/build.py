@@ -30,11 +30,13 @@ HIP_FLAGS = [
 ]
 
 
-# Per-source extra flags. The ring GEMM and the column-block kernel keep their MFMA results in
+# Per-source extra flags. The ring and wide GEMMs and the column-block kernel keep their MFMA results in
 # ordinary VGPRs (the VALU fix-up reads every one; in accumulation registers each read costs a
 # copy).
-FILE_FLAGS = {"affine_gemm_ring.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-              "affine_qmv_block.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+_WIDE = [f"affine_wide_{name}.hip" for name in ("u4_bf16", "u4_f16", "u8_bf16", "u8_f16",
+                                                "u8g32_bf16", "u8g32_f16")]
+FILE_FLAGS = {name: _VGPR_FORM for name in ("affine_gemm_ring.hip", "affine_qmv_block.hip", *_WIDE)}
 
 
 def hipcc() -> str:

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
@@ -19,6 +20,7 @@
 #include "dense_qmv.h"
 #include "affine_gemm.h"
 #include "affine_quantize.h"
+#include "affine_wide.h"
 #include "stream_read.h"
 
 namespace {
@@ -257,7 +259,7 @@ struct PlanKeyHash {
   }
 };
 
-enum PlanOp : int { kOpQmv = 0, kOpGemm = 1, kOpDense = 2 };
+enum PlanOp : int { kOpQmv = 0, kOpGemm = 1, kOpDense = 2, kOpWide = 3 };
 
 std::shared_mutex g_plans_mu;
 std::unordered_map<PlanKey, mt_qmv_plan, PlanKeyHash> g_qmv_plans;
@@ -576,6 +578,158 @@ void set_layout(mt::QmvParams& p, int layout, int bits) {
   }
 }
 
+// ---- calls of more rows than one small-row dispatch: the wide kernel (affine_wide.hip) ------------
+
+struct WidePlan {
+  int tile_m, tile_n, ksplit, steps_per_split;
+  int tiles;
+};
+
+WidePlan make_wide(int M, int K, int N, int nproj, int group_size, int tile_m, int tile_n,
+                   int ksplit) {
+  WidePlan w{};
+  w.tile_m = tile_m;
+  w.tile_n = tile_n;
+  w.tiles = ((M + tile_m - 1) / tile_m) * ((N * nproj + tile_n - 1) / tile_n);
+  const int steps = K / 64, unit = mt::wide_split_unit(group_size);
+  const int len = (steps + ksplit - 1) / ksplit;
+  w.steps_per_split = (len + unit - 1) / unit * unit;
+  w.ksplit = (steps + w.steps_per_split - 1) / w.steps_per_split;
+  return w;
+}
+
+size_t wide_bytes(const WidePlan& w) {
+  return w.ksplit > 1 ? kCounterBytes + (size_t)w.ksplit * w.tiles *
+                                            mt::wide_part_bytes(w.tile_m, w.tile_n)
+                      : 0;
+}
+
+// Microseconds a wide launch is expected to take: a fit (rms error 10%) to 2772 measured (shape,
+// plan) pairs on MI355X, 24 to 2048 rows, K 896 to 14336, N 896 to 17408, one and two projections;
+// the plan it picks was on average 2.3% behind the best of its shape. A CU holds eight waves at a
+// time (LDS and registers): a workgroup of eight, two of four (one with 128 rows), three of two.
+// Each batch pays a start and end (loads, the bias products, stores) and its K steps, whose cost
+// grows with the rows and, shared with other waves, with the waves resident; a K split pays its
+// partial sums' way through memory; the launch cannot be faster than its weights arrive.
+double wide_cost(int M, int K, int N, int nproj, int group_size, int bits, const WidePlan& w) {
+  constexpr double kLaunch = 2.3, kPerWg = 0.00076;
+  const int cus = device_cus();
+  const int row_tiles = w.tile_m / 32;
+  const int resident = w.tile_n == 256 ? 1 : w.tile_n == 128 ? (w.tile_m == 128 ? 1 : 2)
+                                                             : (w.tile_m <= 64 ? 3 : 2);
+  const long wgs = (long)w.tiles * w.ksplit;
+  const long load = (wgs + cus - 1) / cus;  // on the busiest CU
+  const double steps = (w.steps_per_split + 3) / 4 * 4;
+  const double slow = 1.0 + (bits == 8 ? 0.16 : 0.0) + (group_size == 32 ? 0.98 : 0.0) +
+                      (w.tile_n == 64 ? 0.20 : 0.0);
+  auto batch = [&](long b) {
+    const double full = b * w.tile_n / 256.0;  // share of the CU's waves
+    return 1.5 + 1.03 * row_tiles * full +
+           steps * slow * (0.05 + 0.11 * row_tiles + full * (0.25 + 0.046 * row_tiles));
+  };
+  double us = kLaunch + kPerWg * wgs + (load / resident) * batch(resident);
+  if (load % resident) us += batch(load % resident);
+  if (w.ksplit > 1)
+    us += 2.0 + 0.29 * w.ksplit * row_tiles + 0.74e-6 * w.ksplit * M * ((double)N * nproj);
+  const double read = 0.33e-6 * N * (double)K * nproj * (bits / 8.0 + 4.0 / group_size);
+  return std::sqrt(us * us + read * read);
+}
+
+WidePlan search_wide(int M, int K, int N, int nproj, int group_size, int bits) {
+  WidePlan best{};
+  double best_us = 0.0;
+  for (int tile_m : {32, 64, 96, 128}) {
+    if (tile_m > 32 && M <= tile_m - 32) break;  // a whole row tile would be empty
+    for (int tile_n : {64, 128, 256})
+      for (int ksplit : {1, 2, 3, 4, 6, 8, 12}) {
+        if (ksplit > 1 && K / 64 < 4 * ksplit) break;
+        const WidePlan w = make_wide(M, K, N, nproj, group_size, tile_m, tile_n, ksplit);
+        // Split: an arrival counter per tile and wave, and 32-bit offsets of the partial sums.
+        if (w.ksplit > 1 && (w.tiles * (tile_n / 32) > kMaxStrips ||
+                             wide_bytes(w) >= (1ull << 31)))
+          continue;
+        const double us = wide_cost(M, K, N, nproj, group_size, bits, w);
+        if (best.tiles == 0 || us < best_us) {
+          best = w;
+          best_us = us;
+        }
+      }
+  }
+  return best;
+}
+
+// The wide kernel's plan for a call, if it takes the call's format and sizes. A thread keeps the last
+// plans it searched (a search costs a few microseconds), in a table of fixed size.
+bool plan_wide(int M, int K, int N, int nproj, int group_size, int bits, WidePlan* out) {
+  if (bits == 4 && group_size < 64) return false;
+  if ((size_t)M * K * 2 >= (1ull << 31) || (size_t)M * N * 2 >= (1ull << 31)) return false;
+  struct Entry {
+    PlanKey key;
+    int device;
+    WidePlan plan;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry table[kEntries] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) device = -1;
+  const PlanKey key{kOpWide, M, K, N, nproj, group_size, bits, 0};
+  Entry& e = table[PlanKeyHash{}(key) % kEntries];
+  if (!(e.key == key) || e.device != device)
+    e = Entry{key, device, search_wide(M, K, N, nproj, group_size, bits)};
+  *out = e.plan;
+  return true;
+}
+
+// Workspace with which a small-row entry's call of M rows takes the wide kernel (0: it needs none, or
+// the call is not one that it takes).
+size_t rows_workspace(int M, int K, int N, int nproj, int group_size, int bits) {
+  WidePlan w;
+  if (M <= row_chunk(group_size) || !plan_wide(M, K, N, nproj, group_size, bits, &w)) return 0;
+  return wide_bytes(w);
+}
+
+// Whether a call of this shape takes the wide kernel, given its workspace.
+bool use_wide(int M, int K, int N, int nproj, int group_size, int bits, const void* workspace,
+              size_t workspace_bytes, WidePlan* out) {
+  if (!plan_wide(M, K, N, nproj, group_size, bits, out)) return false;
+  const size_t need = wide_bytes(*out);
+  return need == 0 || (workspace && workspace_bytes >= need);
+}
+
+int run_wide(const char* op, const WidePlan& plan, int nproj, const void* x,
+             const uint32_t* const w[2], const void* const s[2], const void* const b[2],
+             const void* residual, void* y, int M, int K, int N, int group_size, int bits, int dtype,
+             void* workspace, void* stream, int layout) {
+  mt::WideParams p{};
+  p.x = static_cast<const uint16_t*>(x);
+  for (int q = 0; q < 2; ++q) {
+    const int src = q < nproj ? q : 0;
+    p.w[q] = w[src];
+    p.s[q] = static_cast<const uint16_t*>(s[src]);
+    p.b[q] = static_cast<const uint16_t*>(b[src]);
+  }
+  p.residual = static_cast<const uint16_t*>(residual);
+  p.y = static_cast<uint16_t*>(y);
+  if (plan.ksplit > 1) {
+    p.counters = static_cast<uint32_t*>(workspace);
+    p.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
+  }
+  p.M = M;
+  p.K = K;
+  p.N = N;
+  p.group_shift = __builtin_ctz((unsigned)group_size);
+  p.tile_m = plan.tile_m;
+  p.tile_n = plan.tile_n;
+  p.ksplit = plan.ksplit;
+  p.steps_per_split = plan.steps_per_split;
+  p.col_stride = layout == kLayoutStepMajor ? 8u * (uint32_t)bits : (uint32_t)K * (uint32_t)bits / 8u;
+  p.step_stride = layout == kLayoutStepMajor ? (uint32_t)N * 8u * (uint32_t)bits : 8u * (uint32_t)bits;
+  const hipError_t e =
+      mt::launch_affine_wide(p, bits, dtype, nproj, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, op);
+  return MT_OK;
+}
+
 int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2],
             const void* const s[2], const void* const b[2], const void* residual, void* y,
             int M, int K, int N, int group_size, int bits, int dtype, void* workspace,
@@ -587,12 +741,16 @@ int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2]
     if (!w[q] || !s[q] || !b[q])
       return fail(MT_ERR_INVALID_ARGUMENT,
                   std::string(op) + ": null packed weight, scales or biases");
+  const int chunk = row_chunk(group_size);
+  WidePlan wide;
+  if (M > chunk && use_wide(M, K, N, nproj, group_size, bits, workspace, workspace_bytes, &wide))
+    return run_wide(op, wide, nproj, x, w, s, b, residual, y, M, K, N, group_size, bits, dtype,
+                    workspace, stream, layout);
   const size_t need = qmv_workspace(M, K, N, nproj, group_size, bits);
   if (need && (!workspace || workspace_bytes < need))
     return fail(MT_ERR_WORKSPACE, std::string(op) + ": workspace of " + std::to_string(need) +
                                       " bytes required, got " + std::to_string(workspace_bytes));
   const hipStream_t hs = static_cast<hipStream_t>(stream);
-  const int chunk = row_chunk(group_size);
   for (int r0 = 0; r0 < M; r0 += chunk) {
     const int rows = (M - r0) < chunk ? (M - r0) : chunk;
     const Plan plan = plan_qmv(rows, K, N, nproj, group_size, bits, dtype);
@@ -997,9 +1155,12 @@ struct MlpPlan {
   size_t hidden, bytes;  // workspace offset of the hidden activation, and the total
 };
 
-MlpPlan plan_mlp(int M, int H, int I, int group_size, int bits) {
-  const size_t a = qmv_workspace(M, H, I, 2, group_size, bits);
-  const size_t b = qmv_workspace(M, I, H, 1, group_size, bits);
+// `rows`: with room for the wide kernel's split K, where the call is one that it takes.
+MlpPlan plan_mlp(int M, int H, int I, int group_size, int bits, bool rows) {
+  const size_t a = std::max(qmv_workspace(M, H, I, 2, group_size, bits),
+                            rows ? rows_workspace(M, H, I, 2, group_size, bits) : 0);
+  const size_t b = std::max(qmv_workspace(M, I, H, 1, group_size, bits),
+                            rows ? rows_workspace(M, I, H, 1, group_size, bits) : 0);
   const size_t split = align_up(a > b ? a : b);
   MlpPlan mp{};
   mp.hidden = split > kCounterBytes ? split : kCounterBytes;
@@ -1054,7 +1215,9 @@ int affine_mlp_impl(const char* op, const void* x, const uint32_t* gate_w,
                     int down_layout) {
   int st = mlp_check_shape(op, M, H, I, group_size, bits, dtype);
   if (st) return st;
-  const size_t need = plan_mlp(M, H, I, group_size, bits).bytes;
+  MlpPlan mp = plan_mlp(M, H, I, group_size, bits, true);
+  if (workspace_bytes < mp.bytes) mp = plan_mlp(M, H, I, group_size, bits, false);
+  const size_t need = mp.bytes;
   if (!workspace || workspace_bytes < need)
     return fail(MT_ERR_WORKSPACE, std::string(op) + ": workspace of " + std::to_string(need) +
                                       " bytes required, got " + std::to_string(workspace_bytes));
@@ -1062,7 +1225,6 @@ int affine_mlp_impl(const char* op, const void* x, const uint32_t* gate_w,
                                up_biases, down_w, down_scales, down_biases};
   st = mlp_check_pointers(op, x, y, ptrs);
   if (st) return st;
-  const MlpPlan mp = plan_mlp(M, H, I, group_size, bits);
   void* h = static_cast<char*>(workspace) + mp.hidden;
   st = affine_swiglu_impl(op, x, gate_w, gate_scales, gate_biases, up_w, up_scales, up_biases, h,
                           M, H, I, group_size, bits, dtype, workspace, mp.hidden, stream,
@@ -1084,7 +1246,7 @@ size_t affine_mlp_workspace(int M, int H, int I, int group_size, int bits) {
   if (check_affine("mt_affine_mlp", M, H, I, group_size, bits, MT_BF16) ||
       check_affine("mt_affine_mlp", M, I, H, group_size, bits, MT_BF16))
     return 0;
-  return plan_mlp(M, H, I, group_size, bits).bytes;
+  return plan_mlp(M, H, I, group_size, bits, false).bytes;
 }
 
 int affine_mlp_check(const char* op, const void* x, const uint32_t* gate_w,
@@ -1144,7 +1306,19 @@ size_t mt_affine_mlp_workspace_bytes(int M, int H, int I, int group_size, int bi
   if (check_affine("mt_affine_mlp_workspace_bytes", M, H, I, group_size, bits, MT_BF16) ||
       check_affine("mt_affine_mlp_workspace_bytes", M, I, H, group_size, bits, MT_BF16))
     return 0;
-  return plan_mlp(M, H, I, group_size, bits).bytes;
+  return plan_mlp(M, H, I, group_size, bits, false).bytes;
+}
+
+size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int bits, int nproj) {
+  if (check_affine("mt_affine_rows_workspace_bytes", M, K, N, group_size, bits, MT_BF16)) return 0;
+  return rows_workspace(M, K, N, nproj == 2 ? 2 : 1, group_size, bits);
+}
+
+size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits) {
+  if (check_affine("mt_affine_mlp_rows_workspace_bytes", M, H, I, group_size, bits, MT_BF16) ||
+      check_affine("mt_affine_mlp_rows_workspace_bytes", M, I, H, group_size, bits, MT_BF16))
+    return 0;
+  return plan_mlp(M, H, I, group_size, bits, true).bytes;
 }
 
 int mt_affine_mlp(const void* x, const uint32_t* gate_w, const void* gate_scales,
@@ -1312,6 +1486,16 @@ int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const
     return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: tensor larger than 2 GiB");
   if (!x || !w_q || !scales || !biases || !y)
     return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: null pointer");
+  mt_gemm_plan installed;
+  WidePlan wide;
+  if (M > kRowChunk && !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
+      use_wide(M, K, N, 1, group_size, bits, workspace, workspace_bytes, &wide)) {
+    const uint32_t* const w[2] = {w_q, nullptr};
+    const void* const s[2] = {scales, nullptr};
+    const void* const b[2] = {biases, nullptr};
+    return run_wide("mt_affine_gemm", wide, 1, x, w, s, b, nullptr, y, M, K, N, group_size, bits,
+                    dtype, workspace, stream, kLayoutMlx);
+  }
   const GemmPlan g = plan_gemm(M, K, N, group_size, dtype);
   const size_t need = gemm_workspace(M, K, N, group_size);
   if (need && (!workspace || workspace_bytes < need))

@@ -15,7 +15,7 @@ constexpr size_t kWorkspaceCounterBytes = 64 * 1024;
 // Records `msg` as the calling thread's last error (mt_last_error) and returns `status`.
 int set_last_error(int status, const std::string& msg);
 
-// Workspace bytes mt_affine_mlp needs at this shape (0 for a shape it rejects).
+// Workspace bytes without which mt_affine_mlp refuses this shape (0 for a shape it rejects).
 size_t affine_mlp_workspace(int M, int H, int I, int group_size, int bits);
 
 // The argument checks of mt_affine_mlp other than the workspace's (shapes, dtype, bits, group

@@ -135,6 +135,18 @@ def _check_params(values, weight, scales, biases, group_size, bits, what):
 # ---------------------------------------------------------------------------------------------
 
 
+_MIN_CHUNK = 16  # rows that every small-row dispatch takes
+
+
+def _qmv_workspace(L, m, k, n, group_size, bits, nproj):
+    """Workspace bytes of a QMV or SwiGLU call: what its dispatches need, and with more rows than
+    one dispatch takes what the wide kernel needs in their place."""
+    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, nproj)
+    if m > _MIN_CHUNK:
+        need = max(need, L.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, nproj))
+    return need
+
+
 def affine_qmv(values, weight, scales, biases, *, group_size=64, bits=4, residual=None):
     """``values @ dequantize(weight).T (+ residual)`` with fp32 accumulation.
 
@@ -164,7 +176,7 @@ def affine_qmv(values, weight, scales, biases, *, group_size=64, bits=4, residua
     s = scales.contiguous()
     b = biases.contiguous()
     L = _lib.lib()
-    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, 1)
+    need = _qmv_workspace(L, m, k, n, group_size, bits, 1)
     ws = workspace(values.device, need) if need else None
     fn = L.mt_affine_qmv_repacked if _repacked(w) else L.mt_affine_qmv
     _lib.check(fn(
@@ -200,7 +212,7 @@ def affine_swiglu(values, gate_weight, gate_scales, gate_biases, up_weight, up_s
     gs, gb = gate_scales.contiguous(), gate_biases.contiguous()
     us, ub = up_scales.contiguous(), up_biases.contiguous()
     L = _lib.lib()
-    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, 2)
+    need = _qmv_workspace(L, m, k, n, group_size, bits, 2)
     ws = workspace(values.device, need) if need else None
     fn = L.mt_affine_swiglu_repacked if _repacked(gw) else L.mt_affine_swiglu
     _lib.check(fn(
@@ -251,7 +263,7 @@ def affine_mlp(values, gate, up, down, *, group_size=64, bits=4, residual=None):
     tensors = [_as_u32(gw), gs.contiguous(), gb.contiguous(), _as_u32(uw), us.contiguous(),
                ub.contiguous(), _as_u32(dw), ds.contiguous(), db.contiguous()]
     L = _lib.lib()
-    need = L.mt_affine_mlp_workspace_bytes(m, hdim, idim, group_size, bits)
+    need = L.mt_affine_mlp_rows_workspace_bytes(m, hdim, idim, group_size, bits)
     ws = workspace(values.device, need)
     args = (x.data_ptr(), *[t.data_ptr() for t in tensors], _ptr(res), out.data_ptr(), m, hdim,
             idim, group_size, bits, code)
@@ -332,7 +344,7 @@ class BoundMlp:
         for attempt in (0, 1):
             need = self.need.get(m) if attempt == 0 else None
             if need is None:  # installed plans may change the need: refreshed on a refusal
-                need = self.need[m] = L.mt_affine_mlp_workspace_bytes(
+                need = self.need[m] = L.mt_affine_mlp_rows_workspace_bytes(
                     m, self.hdim, self.idim, self.group_size, self.bits)
             ws = workspace(self.device, need, stream)
             st = L.mt_affine_mlp_layouts(
@@ -413,7 +425,8 @@ def affine_matmul(values, weight, scales, biases, *, group_size=64, bits=4):
     w = _as_u32(weight)
     s, b = scales.contiguous(), biases.contiguous()
     lib = _lib.lib()
-    need = lib.mt_affine_gemm_workspace_bytes(m, k, n, group_size, bits)
+    need = max(lib.mt_affine_gemm_workspace_bytes(m, k, n, group_size, bits),
+               lib.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, 1))
     ws = workspace(values.device, need) if need else None
     _lib.check(lib.mt_affine_gemm(
         x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), out.data_ptr(), m, k, n,

@@ -773,7 +773,8 @@ def _tune_gemm(values, weight, scales, biases, group_size):
     need = 0
     for plan in [None, *candidates]:
         install_gemm_plan(rows, k, n, group_size, dtype, plan)
-        need = max(need, L.mt_affine_gemm_workspace_bytes(rows, k, n, group_size, 4))
+        need = max(need, L.mt_affine_gemm_workspace_bytes(rows, k, n, group_size, 4),
+                   L.mt_affine_rows_workspace_bytes(rows, k, n, group_size, 4, 1))
     install_gemm_plan(rows, k, n, group_size, dtype, None)
     bench = _Bench(values.device, need)
     x = values.contiguous()

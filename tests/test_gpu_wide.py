@@ -1,0 +1,144 @@
+"""Calls of more rows than one small-row dispatch takes, through the entry points: the wide kernel's
+tile edges (rows and columns beside multiples of 32, 64, 96 and 128), one K step and step counts
+beside its four- and eight-step loop and its 16-group chunks, odd group counts (scale rows that start
+inside a dword), K splits, both code widths, all group sizes, both types, both layouts, residuals and
+the SwiGLU epilogue, against the oracle.
+
+The bars are the contract's: 2e-3 of the largest output after removing the final rounding, and at
+least 98% (bf16) or 90% (f16) of outputs equal to the correctly rounded reference."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import metile_amd as mt
+from metile_amd import _lib
+from oracle import affine as O
+from tests.helpers import act_to_torch, affine_to_torch, torch_to_act
+
+TOL = 2e-3
+
+# rows, K, N, bits, group, dtype, projections, residual, repacked
+CASES = [
+    (33, 64, 32, 4, 64, "bf16", 1, False, False),       # one K step, one column block
+    (33, 320, 96, 4, 64, "f16", 1, True, True),         # five steps, odd groups a row
+    (64, 1088, 288, 4, 64, "bf16", 1, True, False),     # 17 groups: a chunk and one more
+    (65, 1024, 256, 4, 128, "f16", 1, False, True),
+    (96, 2112, 96, 4, 64, "bf16", 2, False, False),     # SwiGLU, 33 groups
+    (97, 768, 160, 4, 256, "bf16", 2, False, True),
+    (128, 1536, 1024, 4, 64, "bf16", 1, True, True),
+    (129, 1536, 320, 4, 64, "f16", 2, False, False),
+    (300, 576, 544, 4, 64, "bf16", 1, False, False),
+    (48, 8960, 192, 4, 64, "bf16", 1, True, False),     # few columns, long K: K splits
+    (40, 4096, 64, 4, 128, "f16", 1, True, True),
+    (17, 64, 32, 8, 32, "bf16", 1, False, False),       # groups of 32 leave small rows at 16
+    (40, 544 * 2, 96, 8, 32, "f16", 2, False, True),    # 34 groups of 32
+    (64, 640, 128, 8, 64, "bf16", 2, False, False),
+    (100, 1152, 96, 8, 128, "f16", 1, True, False),
+    (130, 2048, 288, 8, 32, "bf16", 1, True, True),
+    (36, 5120, 64, 8, 64, "f16", 1, False, True),       # K splits
+]
+
+
+def _fn(nproj, repacked):
+    lib = _lib.lib()
+    if nproj == 2:
+        return lib.mt_affine_swiglu_repacked if repacked else lib.mt_affine_swiglu
+    return lib.mt_affine_qmv_repacked if repacked else lib.mt_affine_qmv
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,bits,g,dtype,nproj,residual,repacked", CASES)
+def test_wide_meets_the_contract(m, k, n, bits, g, dtype, nproj, residual, repacked):
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    print(f"[wide] {m}x{k}x{n} bits={bits} g={g} {dtype} nproj={nproj}", flush=True)
+    x = O.make_activations(m, k, 51, dtype=dtype)
+    res = O.make_activations(m, n, 51, tensor_id=3, dtype=dtype) if residual else None
+    weights = [O.make_affine_weight(n, k, bits, g, 51, 10 + 2 * p, dtype=dtype)
+               for p in range(nproj)]
+    xt = act_to_torch(x, dtype)
+    triples = [affine_to_torch(w, dtype) for w in weights]
+    if repacked:
+        triples = [(mt.affine_repack(w, bits=bits), s, b) for w, s, b in triples]
+    if nproj == 2:
+        ref = O.affine_swiglu(x, *weights, g, bits, dtype=dtype)
+        got = mt.affine_swiglu(xt, *triples[0], *triples[1], group_size=g, bits=bits)
+    else:
+        rt = act_to_torch(res, dtype) if residual else None
+        ref = O.affine_qmv(x, *weights[0], g, bits, dtype=dtype, residual=res)
+        got = mt.affine_qmv(xt, *triples[0], group_size=g, bits=bits, residual=rt)
+    y = torch_to_act(got, dtype)
+    err = O.tolerance_error(y, ref, dtype)
+    rounded = O.to_f32(O.from_f32(ref.astype(np.float32), dtype), dtype)
+    same = np.mean(O.to_f32(y, dtype) == rounded)
+    print(f"[wide] tolerance_error={err:.2e} exact={same:.5f}", flush=True)
+    assert err <= TOL and same >= (0.98 if dtype == "bf16" else 0.90)
+    # with the sizes of the row dispatches the call runs as before (the same contract)
+    lib = _lib.lib()
+    need = lib.mt_affine_qmv_workspace_bytes(m, k, n, g, bits, nproj)
+    ws = torch.zeros(max(need, 1), dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(got)
+    args = [xt.data_ptr(), *(t.data_ptr() for triple in triples for t in triple)]
+    if nproj == 1:
+        args.append(act_to_torch(res, dtype).data_ptr() if residual else None)
+    keep = act_to_torch(res, dtype) if residual else None
+    if residual:
+        args[-1] = keep.data_ptr()
+    _lib.check(_fn(nproj, repacked)(
+        *args, out.data_ptr(), m, k, n, g, bits, _lib.MT_BF16 if dtype == "bf16" else _lib.MT_F16,
+        ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream))
+    assert O.tolerance_error(torch_to_act(out, dtype), ref, dtype) <= TOL
+
+
+@pytest.mark.gpu
+def test_wide_reads_both_layouts_alike_and_replays_in_a_graph():
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    h, i, m = 512, 4096, 70
+    weights = [affine_to_torch(O.make_affine_weight(n, k, 4, 64, 52, 10 + 2 * p), "bf16")
+               for p, (n, k) in enumerate(((i, h), (i, h), (h, i)))]
+    packed = [(mt.affine_repack(w, bits=4), s, b) for w, s, b in weights]
+    x = act_to_torch(O.make_activations(m, h, 52), "bf16")
+    r = act_to_torch(O.make_activations(m, h, 52, tensor_id=3), "bf16")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = mt.affine_mlp(x, *weights, residual=r)
+        other = mt.affine_mlp(x, *packed, residual=r)
+    side.synchronize()
+    assert torch.equal(want.view(torch.int16), other.view(torch.int16))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = mt.affine_mlp(x, *packed, residual=r)
+    for _ in range(3):
+        got.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_wide_workspace_sizes():
+    """No device: few rows need nothing, the MLP's size covers its stages and the older query, and
+    formats and sizes that the kernel does not take ask for nothing."""
+    lib = _lib.lib()
+    assert lib.mt_affine_rows_workspace_bytes(32, 8960, 1536, 64, 4, 1) == 0
+    split = lib.mt_affine_rows_workspace_bytes(48, 8960, 1536, 64, 4, 1)
+    assert split > 64 * 1024  # few columns, long K: split
+    assert lib.mt_affine_rows_workspace_bytes(48, 8960, 1536, 32, 4, 1) == 0  # 4-bit groups of 32
+    assert lib.mt_affine_rows_workspace_bytes(1 << 20, 8960, 1536, 64, 4, 1) == 0  # x beyond 2 GiB
+    for m in (1, 32, 48, 333):
+        whole = lib.mt_affine_mlp_rows_workspace_bytes(m, 1536, 8960, 64, 4)
+        assert whole >= lib.mt_affine_mlp_workspace_bytes(m, 1536, 8960, 64, 4)
+        assert whole >= (lib.mt_affine_rows_workspace_bytes(m, 8960, 1536, 64, 4, 1)
+                         + m * 8960 * 2)
+    assert (lib.mt_affine_mlp_rows_workspace_bytes(32, 1536, 8960, 64, 4)
+            == lib.mt_affine_mlp_workspace_bytes(32, 1536, 8960, 64, 4))
+    buf = ctypes.c_void_p(256)  # never dereferenced: too small a workspace is refused as before
+    st = lib.mt_affine_mlp(*([buf] * 10), None, buf, 48, 1536, 8960, 64, 4, 0, buf, 1 << 10, None)
+    assert st == _lib.MT_ERR_WORKSPACE
