@@ -330,12 +330,14 @@ affine_wide_kernel(const WideParams args) {
   each(each, IntConst<0>{}, [&](auto ic) {
     constexpr int I = decltype(ic)::value;
     if constexpr (I < DA) {
+      __builtin_amdgcn_sched_barrier(0);
       issue_a(s_beg + I, ic);
       issue_codes(s_beg + I + DC - DA, IntConst<I + DC - DA>{});
     }
   });
-  // In flight behind the first step's activations: the other stages' and the codes issued since.
-  wait_vmcnt<(DA - 1) * kPer + kCodeLoads>();
+  // In flight behind the first step's loads: the other stages'. Within a step the scheduler orders
+  // loads as it likes (they write different memory), so a wait counts whole steps only.
+  wait_vmcnt<(DA - 1) * kPer>();
   sync();
   u32x4 af[2][4], bf[2][4];
   read_a(IntConst<0>{}, 0, af[0]);
@@ -391,7 +393,7 @@ affine_wide_kernel(const WideParams args) {
       } else {
         // Every operand of this step is in registers (or arrives at the wait below): the stage may
         // be refilled behind the barrier, and the next step's stage is complete there.
-        constexpr int kBehind = (DA - 2) * kPer + kCodeLoads;  // since the next step's
+        constexpr int kBehind = (DA - 2) * kPer;  // issued in the steps since the next one's
         if (S > 0 && S < DA - 1 && burst) wait_vmcnt<kBehind + kSbPer>();
         else wait_vmcnt<kBehind>();
         sync();

@@ -142,3 +142,19 @@ def test_wide_workspace_sizes():
     buf = ctypes.c_void_p(256)  # never dereferenced: too small a workspace is refused as before
     st = lib.mt_affine_mlp(*([buf] * 10), None, buf, 48, 1536, 8960, 64, 4, 0, buf, 1 << 10, None)
     assert st == _lib.MT_ERR_WORKSPACE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n", [(40, 1536, 8960), (64, 1536, 2048), (129, 1024, 4096)])
+def test_wide_repeats_to_the_bit(m, k, n):
+    """Short K on a full chip, where the first steps' loads arrive last: every call and both layouts
+    give the same bits (a wait that ends before the loads it counts shows here)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    w = affine_to_torch(O.make_affine_weight(n, k, 4, 64, 53, 10), "bf16")
+    packed = mt.affine_repack(w[0], bits=4)
+    x = act_to_torch(O.make_activations(m, k, 53, dtype="bf16"), "bf16")
+    want = mt.affine_qmv(x, *w, group_size=64, bits=4)
+    for _ in range(20):
+        assert torch.equal(mt.affine_qmv(x, *w, group_size=64, bits=4), want)
+        assert torch.equal(mt.affine_qmv(x, packed, w[1], w[2], group_size=64, bits=4), want)
