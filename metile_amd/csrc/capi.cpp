@@ -125,7 +125,7 @@ int staged_ring(int bits, int nproj, int group_size) {
 // workgroups per CU) are rebalanced: a grid of several rounds evens out as workgroups
 // retire. (Changing the K split instead also measured slower: every split adds a partial-sum
 // hand-off.)
-Plan planner_qmv(int rows, int K, int N, int nproj, int group_size, int bits) {
+Plan planner_strips(int rows, int K, int N, int nproj, int group_size, int bits) {
   Plan plan = plan_split(K, N);
   if (group_size == 32) {
     // Two groups per K step: split K until the staged kernel's scale rows and LDS take it.
@@ -418,12 +418,109 @@ std::string qmv_plan_problem(int rows, int K, int N, int nproj, int group_size, 
   return "";
 }
 
+// Where another kernel than the strip kernels above is the better one in both code layouts (a plan
+// serves both), its plan; else false. Measured over ten (K, N) from 896 x 4864 to 17408 x 5120, cold
+// weights, times against the strip plan's as geometric means (MLX rows, repacked):
+//  * 4-bit codes, one or two rows, K up to 12288 (24 rounds of 512, at most three a wave): the
+//    4x4x4-MFMA GEMV with as many waves as rounds allow and the widest column groups that leave about
+//    two workgroups per CU. Both layouts together take 0.75 / 0.78 of the time with one projection
+//    at one / two rows, 0.76 / 0.78 with two (1536 -> 8960 gate and up at one row 9.5 -> 6.5 and 7.5
+//    -> 6.1 us). Longer K spends more rounds a wave than its loads hide (14336 -> 4096, repacked, at
+//    one row 11.4 -> 14 us).
+//  * 4-bit codes, three or four rows: the same from K = 4096 on, three workgroups for four CUs
+//    (4096 -> 14336 gate and up 33.0 -> 20.7 and 21.5 -> 20.0 us, 4864 -> 896 6.0 -> 4.2 and 5.9 ->
+//    4.1 us); below, repacked codes ran up to 1.1 times as long (2048 -> 8192 6.9 -> 7.5 us).
+//  * 8-bit codes, one or two rows, K up to 8192: the GEMV of four-column groups, one or two passes
+//    over K, groups dealt out XCD by XCD (5120 -> 17408 at one row 47.2 -> 17.6 and 28.7 -> 25.2 us;
+//    together 0.69 at one row, 0.79 at two).
+//  * 8-bit codes in groups of 64 or more, other rows, N of 2048 or more: column blocks of about 32
+//    columns, one or two per CU, K in four splits beyond 96 steps (5120 -> 17408 at 16 rows 52.3 ->
+//    35.8 and 33.7 -> 26.4 us; 14336 -> 4096 at 8 rows 37.8 -> 21.0 and 25.1 -> 16.4 us). Fewer
+//    columns leave CUs idle (8960 -> 1536 at 16 rows 10.3 -> 10.9 us).
+bool preferred_qmv(int rows, int K, int N, int nproj, int group_size, int bits, mt_qmv_plan* out) {
+  const int cus = device_cus();
+  mt_qmv_plan q{};
+  q.ksplit = 1;
+  if (bits == 4) {
+    const int rounds = (K + 511) / 512;
+    if (rows > 4 || rounds > 24 || (rows > 2 && rounds < 8)) return false;
+    int per_wave = 1;
+    while ((rounds + per_wave - 1) / per_wave > mt::kGemv4MaxWaves) ++per_wave;
+    q.kernel = MT_QMV_GEMV4;
+    q.tiles = (rounds + per_wave - 1) / per_wave;
+    const int least = rows > 2 ? cus * 3 / 4 : nproj == 1 ? 2 * cus : 2 * cus + cus / 3;
+    for (int groups : {4, 2, 1}) {
+      if (N % (4 * groups)) continue;
+      q.strips = N / (4 * groups);
+      if (q.strips >= least &&
+          qmv_plan_problem(row_bucket(rows), K, N, nproj, group_size, bits, q).empty())
+        break;
+    }
+  } else if (rows <= 2 && K <= 8192) {
+    const int chunks = K * bits / 128;  // 16-byte code chunks of a column
+    int waves = 1;
+    for (int passes = 1; chunks > 64; ++passes) {
+      waves = (chunks + 64 * passes - 1) / (64 * passes);
+      if (waves <= mt::kGemvMaxWaves) break;
+    }
+    q.kernel = MT_QMV_GEMV;
+    q.tiles = waves;
+    q.order = 1;
+    const int groups = mt::affine_gemv_groups(K, bits, waves);
+    for (int cols : {4, 2}) {
+      if (N % (cols * groups)) continue;
+      q.strips = N / (cols * groups);
+      if (qmv_plan_problem(row_bucket(rows), K, N, nproj, group_size, bits, q).empty()) break;
+    }
+  } else if (group_size >= 64 && N >= 2048) {
+    q.kernel = MT_QMV_BLOCK;
+    q.ksplit = K / 64 <= 96 ? 1 : 4;
+    q.strips = N / 32;
+    if (q.ksplit == 1 && q.strips > cus)
+      q.strips = nproj == 1 && N <= 36 * cus ? cus : N <= 36 * 2 * cus ? 2 * cus : q.strips;
+    q.tiles = q.ksplit == 4 ? 4 : rows > 16 ? 4 : nproj == 1 ? 8 : 6;
+  } else {
+    return false;
+  }
+  *out = q;
+  return qmv_plan_problem(row_bucket(rows), K, N, nproj, group_size, bits, q).empty();
+}
+
+// The planner's plan for dispatches of `rows` rows, and the most K splits of it and the strip
+// kernels' plan (their workspaces). A thread keeps the last plans it made, in a table of fixed size:
+// a call needs its plan several times, and making one costs about a microsecond.
+struct Planned {
+  Plan plan;
+  int splits;
+};
+
+Planned planner_qmv(int rows, int K, int N, int nproj, int group_size, int bits) {
+  struct Entry {
+    PlanKey key;
+    int cus;
+    Planned planned;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry table[kEntries] = {};
+  const PlanKey key{kOpQmv, rows, K, N, nproj, group_size, bits, 0};
+  const int cus = device_cus();
+  Entry& e = table[PlanKeyHash{}(key) % kEntries];
+  if (!(e.key == key) || e.cus != cus) {
+    const Plan strips = planner_strips(rows, K, N, nproj, group_size, bits);
+    mt_qmv_plan q;
+    const Plan plan = preferred_qmv(rows, K, N, nproj, group_size, bits, &q) ? from_public(q, K)
+                                                                             : strips;
+    e = Entry{key, cus, {plan, std::max(plan.ksplit, strips.ksplit)}};
+  }
+  return e.planned;
+}
+
 // The plan dispatches of `rows` rows take: the installed one for the shape, else the planner's.
 Plan plan_qmv(int rows, int K, int N, int nproj, int group_size, int bits, int dtype) {
   mt_qmv_plan q;
   if (find_qmv_plan(qmv_key(rows, K, N, nproj, group_size, bits, dtype), &q))
     return from_public(q, K);
-  return planner_qmv(rows, K, N, nproj, group_size, bits);
+  return planner_qmv(rows, K, N, nproj, group_size, bits).plan;
 }
 
 // Staged strip counts worth measuring at a K split: N / 32, and the counts that put a whole
@@ -516,22 +613,20 @@ std::vector<mt_qmv_plan> qmv_candidates(int rows, int K, int N, int nproj, int g
 
 size_t qmv_workspace(int M, int K, int N, int nproj, int group_size, int bits) {
   // Row chunks and one remainder chunk may plan differently, and so may each dtype: the size
-  // covers every plan a call of this shape can take.
+  // covers every plan a call of this shape can take (and the strip kernels' plan, so that it
+  // grows with the rows and no caller's saved size becomes too small).
   const int chunk = row_chunk(group_size);
   size_t need = 0;
   for (int rows : {M < chunk ? M : chunk, M % chunk}) {
     if (rows < 1) continue;
-    std::vector<Plan> plans{planner_qmv(rows, K, N, nproj, group_size, bits)};
+    int splits = planner_qmv(rows, K, N, nproj, group_size, bits).splits;
     for (int dtype : {MT_BF16, MT_F16}) {
       mt_qmv_plan q;
       if (find_qmv_plan(qmv_key(rows, K, N, nproj, group_size, bits, dtype), &q))
-        plans.push_back(from_public(q, K));
+        splits = std::max(splits, from_public(q, K).ksplit);
     }
-    for (const Plan& plan : plans) {
-      if (plan.ksplit <= 1) continue;
-      const size_t b = kCounterBytes + (size_t)plan.ksplit * nproj * rows * N * 4;
-      if (b > need) need = b;
-    }
+    if (splits <= 1) continue;
+    need = std::max(need, kCounterBytes + (size_t)splits * nproj * rows * N * 4);
   }
   return need;
 }
@@ -665,17 +760,16 @@ bool plan_wide(int M, int K, int N, int nproj, int group_size, int bits, WidePla
   if ((size_t)M * K * 2 >= (1ull << 31) || (size_t)M * N * 2 >= (1ull << 31)) return false;
   struct Entry {
     PlanKey key;
-    int device;
+    int cus;
     WidePlan plan;
   };
   constexpr int kEntries = 64;
   static thread_local Entry table[kEntries] = {};
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess) device = -1;
+  const int cus = device_cus();
   const PlanKey key{kOpWide, M, K, N, nproj, group_size, bits, 0};
   Entry& e = table[PlanKeyHash{}(key) % kEntries];
-  if (!(e.key == key) || e.device != device)
-    e = Entry{key, device, search_wide(M, K, N, nproj, group_size, bits)};
+  if (!(e.key == key) || e.cus != cus)
+    e = Entry{key, cus, search_wide(M, K, N, nproj, group_size, bits)};
   *out = e.plan;
   return true;
 }
