@@ -61,12 +61,6 @@ __device__ __forceinline__ uint64_t uniform_bits(const void* q) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// 16 bytes a lane from memory straight to LDS (lane l to 16 l behind `to`).
-__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* to,
-                                           uint32_t off, uint32_t uniform_off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)to, 16, off, uniform_off, 0, 0);
-}
-
 typedef const unsigned char __attribute__((address_space(1))) * global_ptr_t;
 
 // silu(gate) * up of two accumulator registers x0, x1 of a tile whose rows of 16 lanes hold gate, up,

@@ -906,12 +906,25 @@ int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2]
 }
 
 constexpr int kDenseRowChunk = 128;  // rows per dense dispatch
-// Within a dispatch, more than kDenseSubChunk rows run as grid chunks of kDenseSubChunk rows
-// (two workgroups per CU instead of one with 128-row tiles); each chunk has its own partial
-// sums (kDenseSubChunk rows) and counters.
+// Within a dispatch, more than kDenseSubChunk rows can run as grid chunks of that many, each with its
+// own partial sums (kDenseSubChunk rows) and counters.
 constexpr int kDenseSubChunk = 64;
 
-int dense_row_chunk(int rows) { return rows > kDenseSubChunk ? kDenseSubChunk : 0; }
+// Rows per chunk of a dispatch, 0 for one chunk. One chunk has the weights delivered once, two bring
+// them to twice as many CUs from one L2. Two projections are chunked where one chunk would leave a
+// quarter of the CUs idle or a second round mostly empty (at 100 rows 2048 -> 5632, 176 strips, 20.2
+// -> 16.2 us, and 1536 -> 8960, 280 strips, 26.9 -> 22.5; not 2048 -> 8192, 256 strips, 20.4 against
+// 20.7, nor 4096 -> 14336, 68.7 against 77.2); one projection up to 64 MiB of weights, which stay in
+// the caches (8192 -> 2048 19.5 -> 16.3, 8192 -> 3072, 50 MB, 34.6 -> 26.6; not 14336 -> 4096,
+// 117 MB, 46.7 against 53.9).
+int dense_row_chunk(int rows, int K, int N, int nproj, int ksplit) {
+  if (rows <= kDenseSubChunk) return 0;
+  if (nproj == 1) return (size_t)K * N * 2 <= (64u << 20) ? kDenseSubChunk : 0;
+  const int cus = device_cus();
+  const long tiles = (long)(N / 32) * ksplit;
+  const bool idle = tiles * 4 < cus * 3L, tail = tiles > cus && tiles * 4 <= cus * 5L;
+  return idle || tail ? kDenseSubChunk : 0;
+}
 
 // Dense plans: the K split of every dispatch of a (K, N) shape. Keyed without the rows, so that
 // one plan serves every row count and each row keeps its summation order whatever M is (the
@@ -964,8 +977,8 @@ size_t dense_workspace(int M, int K, int N, int nproj) {
   }
   if (ksplit <= 1) return 0;
   const int rows = M < kDenseRowChunk ? M : kDenseRowChunk;
-  const int sub = dense_row_chunk(rows);
-  const int ws_rows = sub ? (rows + sub - 1) / sub * sub : rows;
+  const int ws_rows =
+      rows > kDenseSubChunk ? (rows + kDenseSubChunk - 1) / kDenseSubChunk * kDenseSubChunk : rows;
   return kCounterBytes + (size_t)ksplit * nproj * ws_rows * N * 4;
 }
 
@@ -1016,7 +1029,7 @@ int run_dense(const char* op, int nproj, const void* x, const void* const w[2],
     p.N = N;
     p.ksplit = plan.ksplit;
     p.steps_per_split = plan.steps_per_split;
-    p.row_chunk = dense_row_chunk(rows);
+    p.row_chunk = dense_row_chunk(rows, K, N, nproj, plan.ksplit);
     const hipError_t e = mt::launch_dense_qmv(p, dtype, nproj, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, op);
   }

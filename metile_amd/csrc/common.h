@@ -162,6 +162,13 @@ __device__ __forceinline__ void wait_vmcnt() {
 // LDS address space, for buffer_load...lds destinations.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
+// 16 bytes a lane from memory straight to LDS (lane l to 16 l behind `to`).
+template <int POLICY = 0>
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* to,
+                                           uint32_t off, uint32_t uniform_off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)to, 16, off, uniform_off, 0, POLICY);
+}
+
 // ---- code -> 16-bit float unpack (exact) -------------------------------------------------
 // A 4-bit code q is written into the low mantissa bits of a 16-bit float whose exponent makes
 // the mantissa step exactly 1: bf16 0x4300|q == 128 + q, f16 0x6400|q == 1024 + q. 8-bit

@@ -16,7 +16,7 @@ struct DenseParams {
   int M, K, N;
   int ksplit;
   int steps_per_split;
-  int row_chunk;             // rows per grid z index (rows [z row_chunk, ...) of this launch,
+  int row_chunk;             // 64: rows per grid z index (rows [z row_chunk, ...) of this launch,
                              // each with its own partials and counters); 0: one chunk of M rows
 };
 
