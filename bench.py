@@ -255,6 +255,8 @@ def kernel_label(k, n, nproj):
         flags = f"{str(one_pass).lower()}, {layout}"
         return (f"affine_gemv_kernel<{BITS}, 0, 1, {nproj}, {cols}, {flags}> "
                 f"({plan.strips} workgroups of {waves} waves, {groups} column groups each)")
+    if plan.kernel == "gemv4":
+        return kernel_label_rows(1, k, n, nproj)
     if plan.kernel == "staged":
         return (f"affine_qmv_lds_kernel<{BITS}, 0, 8, {nproj}, ...> "
                 f"({plan.strips} strips, {plan.ksplit} K splits)")
