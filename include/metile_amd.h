@@ -77,8 +77,8 @@ size_t mt_affine_mlp_workspace_bytes(int M, int H, int I, int group_size, int bi
  * of the wide kernel, which reads the weights once per row tile of up to 128 rows, where the format
  * allows (4-bit groups of 64 or more, 8-bit groups of 32 or more; x and y below 2 GiB) and the
  * workspace holds its split-K partials: at least these many bytes. With less they run as row
- * dispatches within the sizes of the queries above. The first is what the wide kernel needs (0 where
- * it does not apply or does not split K), the second at least mt_affine_mlp_workspace_bytes. No
+ * dispatches within the sizes of the queries above. Both cover the sizes of the queries above too
+ * (the first is 0 where the wide kernel does not apply). No
  * counterpart in the reference, whose row kernels loop. */
 size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int bits, int nproj);
 size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits);

@@ -836,14 +836,19 @@ int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2]
       return fail(MT_ERR_INVALID_ARGUMENT,
                   std::string(op) + ": null packed weight, scales or biases");
   const int chunk = row_chunk(group_size);
-  WidePlan wide;
-  if (M > chunk && use_wide(M, K, N, nproj, group_size, bits, workspace, workspace_bytes, &wide))
-    return run_wide(op, wide, nproj, x, w, s, b, residual, y, M, K, N, group_size, bits, dtype,
-                    workspace, stream, layout);
   const size_t need = qmv_workspace(M, K, N, nproj, group_size, bits);
   if (need && (!workspace || workspace_bytes < need))
     return fail(MT_ERR_WORKSPACE, std::string(op) + ": workspace of " + std::to_string(need) +
                                       " bytes required, got " + std::to_string(workspace_bytes));
+  // A call that the row chunks would refuse is refused: the workspace above, and below a group of 32
+  // that no staged plan fits.
+  WidePlan wide;
+  if (M > chunk &&
+      (group_size != 32 ||
+       plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER) &&
+      use_wide(M, K, N, nproj, group_size, bits, workspace, workspace_bytes, &wide))
+    return run_wide(op, wide, nproj, x, w, s, b, residual, y, M, K, N, group_size, bits, dtype,
+                    workspace, stream, layout);
   const hipStream_t hs = static_cast<hipStream_t>(stream);
   for (int r0 = 0; r0 < M; r0 += chunk) {
     const int rows = (M - r0) < chunk ? (M - r0) : chunk;
@@ -1418,7 +1423,10 @@ size_t mt_affine_mlp_workspace_bytes(int M, int H, int I, int group_size, int bi
 
 size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int bits, int nproj) {
   if (check_affine("mt_affine_rows_workspace_bytes", M, K, N, group_size, bits, MT_BF16)) return 0;
-  return rows_workspace(M, K, N, nproj == 2 ? 2 : 1, group_size, bits);
+  const int np = nproj == 2 ? 2 : 1;
+  WidePlan w;
+  if (M <= row_chunk(group_size) || !plan_wide(M, K, N, np, group_size, bits, &w)) return 0;
+  return std::max(wide_bytes(w), qmv_workspace(M, K, N, np, group_size, bits));
 }
 
 size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits) {
@@ -1593,6 +1601,14 @@ int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const
     return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: tensor larger than 2 GiB");
   if (!x || !w_q || !scales || !biases || !y)
     return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: null pointer");
+  const GemmPlan g = plan_gemm(M, K, N, group_size, dtype);
+  const size_t need = gemm_workspace(M, K, N, group_size);
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(MT_ERR_WORKSPACE, "mt_affine_gemm: workspace of " + std::to_string(need) +
+                                      " bytes required, got " + std::to_string(workspace_bytes));
+  if (g.ksplit > 1 && g.tiles > kMaxStrips)
+    return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: too many output tiles to split K");
+  // After the checks: a call of which the plans below would be refused is refused by either kernel.
   mt_gemm_plan installed;
   WidePlan wide;
   if (M > kRowChunk && !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
@@ -1603,13 +1619,6 @@ int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const
     return run_wide("mt_affine_gemm", wide, 1, x, w, s, b, nullptr, y, M, K, N, group_size, bits,
                     dtype, workspace, stream, kLayoutMlx);
   }
-  const GemmPlan g = plan_gemm(M, K, N, group_size, dtype);
-  const size_t need = gemm_workspace(M, K, N, group_size);
-  if (need && (!workspace || workspace_bytes < need))
-    return fail(MT_ERR_WORKSPACE, "mt_affine_gemm: workspace of " + std::to_string(need) +
-                                      " bytes required, got " + std::to_string(workspace_bytes));
-  if (g.ksplit > 1 && g.tiles > kMaxStrips)
-    return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_gemm: too many output tiles to split K");
   mt::GemmParams p{};
   p.x = static_cast<const uint16_t*>(x);
   p.w = w_q;

@@ -144,6 +144,21 @@ def test_wide_workspace_sizes():
     assert st == _lib.MT_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("m,k,n", [(333, 8960, 1536), (2048, 4864, 896), (512, 14336, 4096)])
+def test_wide_refuses_what_the_row_kernels_refuse(m, k, n):
+    """A workspace below the plain queries is refused, also where the wide kernel could do with it."""
+    lib = _lib.lib()
+    buf = ctypes.c_void_p(256)  # never dereferenced
+    need = lib.mt_affine_qmv_workspace_bytes(m, k, n, 64, 4, 1)
+    assert need > 0 and lib.mt_affine_rows_workspace_bytes(m, k, n, 64, 4, 1) >= need
+    assert lib.mt_affine_qmv(buf, buf, buf, buf, None, buf, m, k, n, 64, 4, 0, buf, need - 1,
+                             None) == _lib.MT_ERR_WORKSPACE
+    need = lib.mt_affine_gemm_workspace_bytes(m, k, n, 64, 4)
+    if need:
+        assert lib.mt_affine_gemm(buf, buf, buf, buf, buf, m, k, n, 64, 4, 0, buf, need - 1,
+                                  None) == _lib.MT_ERR_WORKSPACE
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n", [(40, 1536, 8960), (64, 1536, 2048), (129, 1024, 4096)])
 def test_wide_repeats_to_the_bit(m, k, n):
