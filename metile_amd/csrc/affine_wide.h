@@ -37,7 +37,14 @@ constexpr int wide_split_unit(int group_size) {
   return group_size > 256 ? group_size / 64 : 4;
 }
 
-constexpr int kWideMaxSplits = 32;
+// Bytes of one projection's codes: below 2 GiB for every call, but not so the number of its bits, which
+// 32 bits do not hold from 512 MiB of codes on (K is a multiple of 64, so the row's bytes are whole).
+constexpr uint32_t wide_code_bytes(int N, int K, int bits) {
+  return (uint32_t)N * ((uint32_t)K * (uint32_t)bits / 8u);
+}
+static_assert(wide_code_bytes(152064, 3584, 8) == 544997376u, "a vocabulary head in 8 bits");
+static_assert(wide_code_bytes(131072, 8192, 4) == (512u << 20), "in 4 bits, 2^32 bits of codes");
+static_assert(wide_code_bytes(32, (1 << 26) - 64, 8) == (1u << 31) - 2048u, "the largest codes");
 
 // Bytes of one split's partial sums of one tile.
 constexpr size_t wide_part_bytes(int tile_m, int tile_n) { return (size_t)tile_m * tile_n * 4; }

@@ -207,7 +207,7 @@ affine_wide_kernel(const WideParams args) {
   const unsigned char* const c_base =  // SwiGLU: its own projection
       reinterpret_cast<const unsigned char*>(proj ? p.w[1] : p.w[0]) + c_src;
   uint32_t cw[DC][kCodeWords];  // codes of the steps in flight, by stage
-  const uint32_t wbytes = (uint32_t)N * (uint32_t)K * BITS / 8u;
+  const uint32_t wbytes = wide_code_bytes(N, K, BITS);
   // Steps past the end load the last one again (unused).
   auto issue_a = [&](int st, auto sc) {
     const uint32_t at = (uint32_t)min(st, s_end - 1);

@@ -173,3 +173,32 @@ def test_wide_repeats_to_the_bit(m, k, n):
     for _ in range(20):
         assert torch.equal(mt.affine_qmv(x, *w, group_size=64, bits=4), want)
         assert torch.equal(mt.affine_qmv(x, packed, w[1], w[2], group_size=64, bits=4), want)
+
+
+# rows, K, N, bits: codes of 512 MiB and more (a range in bits wraps at 2^32), a vocabulary head
+# among them
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,bits", [(33, 3584, 152064, 8), (40, 8192, 131072, 4)])
+def test_wide_reaches_every_column_of_large_codes(m, k, n, bits):
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    print(f"[wide] {m}x{k}x{n} bits={bits}: {n * k * bits // 8 >> 20} MiB of codes", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(54)
+    words = torch.randint(-2**31, 2**31, (n, k * bits // 32), generator=g, device="cuda",
+                          dtype=torch.int64).to(torch.int32)
+    coef, zero = (0.02, 8.0) if bits == 4 else (0.002, 128.0)
+    scales = (torch.randn(n, k // 64, generator=g, device="cuda").abs() * coef).bfloat16()
+    biases = (scales.float() * -zero).bfloat16()
+    x = O.make_activations(m, k, 54)
+    xt = act_to_torch(x, "bf16")
+    got = [mt.affine_qmv(xt, words, scales, biases, bits=bits),
+           mt.affine_qmv(xt, mt.affine_repack(words, bits=bits), scales, biases, bits=bits)]
+    if bits == 4:
+        got.append(mt.affine_matmul(xt, words, scales, biases))
+    for first in (0, n // 2, n - 64):
+        cols = slice(first, first + 64)
+        ref = O.affine_qmv(x, words[cols].cpu().numpy().view(np.uint32),
+                           torch_to_act(scales[cols], "bf16"), torch_to_act(biases[cols], "bf16"),
+                           64, bits)
+        for y in got:
+            assert O.tolerance_error(torch_to_act(y[:, cols], "bf16"), ref) <= TOL, first
