@@ -21,7 +21,10 @@
  *   dense weights         16-bit floats [N, K]
  * Kernels read x, w_q, dense weights and workspaces with 16-byte loads: these pointers must be
  * 16-byte aligned (allocations are; a row slice of a conforming tensor stays aligned, since
- * K % 64 == 0 and N % 32 == 0). Scales and biases need 4-byte alignment. Nothing checks this.
+ * K % 64 == 0 and N % 32 == 0), and so must mt_affine_gemm's y. Scales and biases need 4-byte
+ * alignment. Nothing refuses other pointers. residual, and y of the other entries, may start at any
+ * element (calls of more than 32 rows whose residual or y is not 4-byte aligned run as dispatches of
+ * up to 32 rows).
  */
 #ifndef METILE_AMD_H
 #define METILE_AMD_H

@@ -654,6 +654,14 @@ int check_affine(const char* op, int M, int K, int N, int group_size, int bits, 
   return MT_OK;
 }
 
+// Whether the kernels for many rows (wide, dense tiles) take these buffers: they bring activations (and
+// dense weights) to LDS 16 bytes a lane and move the residual and the output four bytes at a time, where
+// the row kernels move single elements. Others run on the row kernels.
+bool wide_aligned(const void* x, const void* residual, const void* y) {
+  return ((reinterpret_cast<uintptr_t>(x) & 15u) |
+          ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(y)) & 3u)) == 0;
+}
+
 // Code layouts the small-row kernels read: MLX's output-major words, or the step-major repack
 // of mt_affine_repack.
 enum CodeLayout : int { kLayoutMlx = 0, kLayoutStepMajor = 1 };
@@ -843,7 +851,7 @@ int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2]
   // A call that the row chunks would refuse is refused: the workspace above, and below a group of 32
   // that no staged plan fits.
   WidePlan wide;
-  if (M > chunk &&
+  if (M > chunk && wide_aligned(x, residual, y) &&
       (group_size != 32 ||
        plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER) &&
       use_wide(M, K, N, nproj, group_size, bits, workspace, workspace_bytes, &wide))
@@ -1018,8 +1026,12 @@ int run_dense(const char* op, int nproj, const void* x, const void* const w[2],
     return fail(MT_ERR_WORKSPACE, std::string(op) + ": workspace of " + std::to_string(need) +
                                       " bytes required, got " + std::to_string(workspace_bytes));
   const Plan plan = plan_dense(K, N, nproj, dtype);
-  for (int r0 = 0; r0 < M; r0 += kDenseRowChunk) {
-    const int rows = (M - r0) < kDenseRowChunk ? (M - r0) : kDenseRowChunk;
+  // The kernel of up to 32 rows takes buffers of any alignment, with the same sums.
+  const bool tiles_ok = wide_aligned(x, residual, y) && wide_aligned(w[0], nullptr, nullptr) &&
+                        (nproj == 1 || wide_aligned(w[1], nullptr, nullptr));
+  const int chunk = tiles_ok ? kDenseRowChunk : kRowChunk;
+  for (int r0 = 0; r0 < M; r0 += chunk) {
+    const int rows = (M - r0) < chunk ? (M - r0) : chunk;
     mt::DenseParams p{};
     p.x = static_cast<const uint16_t*>(x) + (size_t)r0 * K;
     for (int q = 0; q < nproj; ++q) p.w[q] = static_cast<const uint16_t*>(w[q]);
@@ -1611,7 +1623,7 @@ int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const
   // After the checks: a call of which the plans below would be refused is refused by either kernel.
   mt_gemm_plan installed;
   WidePlan wide;
-  if (M > kRowChunk && !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
+  if (M > kRowChunk && wide_aligned(x, nullptr, y) && !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
       use_wide(M, K, N, 1, group_size, bits, workspace, workspace_bytes, &wide)) {
     const uint32_t* const w[2] = {w_q, nullptr};
     const void* const s[2] = {scales, nullptr};

@@ -71,3 +71,27 @@ def test_rows_equal_single_row_runs(k, n, nproj, with_residual, dtype):
             if r < m:
                 assert torch.equal(got[r], alone[r]), (m, r)
         assert bool((got[m] == 7.0).all())  # nothing behind the last row
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k,n,nproj", [(320, 64, 2), (576, 160, 1), (4160, 320, 1)])
+def test_residual_and_output_at_an_odd_element(k, n, nproj, dtype):
+    """Neither needs alignment: the same bits as with aligned ones, nothing written beside them."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    m = 100
+    g = torch.Generator(device="cuda").manual_seed(k)
+    weights = [(torch.randn(n, k, generator=g, device="cuda") / k**0.5).to(dtype)
+               for _ in range(nproj)]
+    x = torch.randn(m, k, generator=g, device="cuda").to(dtype)
+    res = torch.randn(m, n, generator=g, device="cuda").to(dtype) if nproj == 1 else None
+    want = _run(x, weights, res, torch.empty(m, n, dtype=dtype, device="cuda"))
+    if nproj == 1:
+        odd = torch.empty(m * n + 1, dtype=dtype, device="cuda")[1:].view(m, n).copy_(res)
+        assert odd.data_ptr() % 4 == 2
+        assert torch.equal(_run(x, weights, odd, torch.empty_like(want)), want)
+    buf = torch.full((m * n + 9,), 7.0, dtype=dtype, device="cuda")
+    got = _run(x, weights, res, buf[1:1 + m * n].view(m, n))
+    assert got.data_ptr() % 4 == 2 and torch.equal(got, want)
+    assert float(buf[0]) == 7.0 and bool((buf[1 + m * n:] == 7.0).all())

@@ -44,6 +44,13 @@ CASES = [
 ]
 
 
+def _shifted(t):
+    """``t`` at an odd element offset of its buffer (2 bytes behind a 16-byte boundary)."""
+    out = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[1:1 + t.numel()].view(t.shape)
+    assert out.data_ptr() % 16 == 2
+    return out.copy_(t)
+
+
 def _fn(nproj, repacked):
     lib = _lib.lib()
     if nproj == 2:
@@ -202,3 +209,33 @@ def test_wide_reaches_every_column_of_large_codes(m, k, n, bits):
                            64, bits)
         for y in got:
             assert O.tolerance_error(torch_to_act(y[:, cols], "bf16"), ref) <= TOL, first
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("repacked", [False, True])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_residual_and_output_at_an_odd_element(dtype, repacked):
+    """They need no alignment: such calls run as row dispatches, bit for bit those of the slices of
+    up to 32 rows, and write nothing beside the output."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    m, k, n = 70, 512, 96
+    x = act_to_torch(O.make_activations(m, k, 55, dtype=dtype), dtype)
+    r = act_to_torch(O.make_activations(m, n, 55, tensor_id=3, dtype=dtype), dtype)
+    w, s, b = affine_to_torch(O.make_affine_weight(n, k, 4, 64, 55, 10, dtype=dtype), dtype)
+    if repacked:
+        w = mt.affine_repack(w, bits=4)
+    want = torch.cat([mt.affine_qmv(x[i:i + 32], w, s, b, residual=r[i:i + 32])
+                      for i in range(0, m, 32)])
+    bits = lambda t: t.contiguous().view(torch.int16)  # noqa: E731
+    assert torch.equal(bits(mt.affine_qmv(x, w, s, b, residual=_shifted(r))), bits(want))
+    lib = _lib.lib()
+    code = _lib.MT_BF16 if dtype == "bf16" else _lib.MT_F16
+    buf = torch.full((m * n + 9,), 7.0, dtype=x.dtype, device="cuda")
+    ws = torch.zeros(1 << 22, dtype=torch.uint8, device="cuda")
+    assert ws.numel() >= lib.mt_affine_rows_workspace_bytes(m, k, n, 64, 4, 1)
+    _lib.check(_fn(1, repacked)(x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(),
+                                r.data_ptr(), buf.data_ptr() + 2, m, k, n, 64, 4, code,
+                                ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(bits(buf[1:1 + m * n].view(m, n)), bits(want))
+    assert float(buf[0]) == 7.0 and bool((buf[1 + m * n:] == 7.0).all())
