@@ -135,16 +135,34 @@ def _check_params(values, weight, scales, biases, group_size, bits, what):
 # ---------------------------------------------------------------------------------------------
 
 
-_MIN_CHUNK = 16  # rows that every small-row dispatch takes
+def _dispatch_rows(group_size):
+    """Most rows of one small-row dispatch."""
+    return 16 if group_size == 32 else 32
 
 
-def _qmv_workspace(L, m, k, n, group_size, bits, nproj):
-    """Workspace bytes of a QMV or SwiGLU call: what its dispatches need, and with more rows than
-    one dispatch takes what the wide kernel needs in their place."""
+def _many_rows_workspace(device, need, least, stream=None):
+    """The workspace of a call: ``need`` bytes, or ``None`` for none. ``least`` (a function) gives
+    what the call's row dispatches need, with which it runs as well, only slower: inside graph
+    capture, where a buffer cannot grow, the buffer that is there is taken if it holds that. (The
+    need does not grow with the rows, so a stream that has run larger calls may lack it.)"""
+    if need and torch.cuda.is_current_stream_capturing():
+        index = device.index if device.index is not None else torch.cuda.current_device()
+        key = (index, _stream_handle(device) if stream is None else stream)
+        with _ws_lock:
+            held = _workspaces.get(key)
+        if held is None or held.numel() < need:
+            need = least()
+    return workspace(device, need, stream) if need else None
+
+
+def _qmv_workspace(L, device, m, k, n, group_size, bits, nproj):
+    """The workspace of a QMV or SwiGLU call: with more rows than one dispatch takes, what the wide
+    kernel needs."""
     need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, nproj)
-    if m > _MIN_CHUNK:
-        need = max(need, L.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, nproj))
-    return need
+    if m <= _dispatch_rows(group_size):
+        return workspace(device, need) if need else None
+    wide = L.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, nproj)
+    return _many_rows_workspace(device, max(need, wide), lambda: need)
 
 
 def affine_qmv(values, weight, scales, biases, *, group_size=64, bits=4, residual=None):
@@ -176,8 +194,7 @@ def affine_qmv(values, weight, scales, biases, *, group_size=64, bits=4, residua
     s = scales.contiguous()
     b = biases.contiguous()
     L = _lib.lib()
-    need = _qmv_workspace(L, m, k, n, group_size, bits, 1)
-    ws = workspace(values.device, need) if need else None
+    ws = _qmv_workspace(L, values.device, m, k, n, group_size, bits, 1)
     fn = L.mt_affine_qmv_repacked if _repacked(w) else L.mt_affine_qmv
     _lib.check(fn(
         x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), _ptr(res), out.data_ptr(),
@@ -212,14 +229,22 @@ def affine_swiglu(values, gate_weight, gate_scales, gate_biases, up_weight, up_s
     gs, gb = gate_scales.contiguous(), gate_biases.contiguous()
     us, ub = up_scales.contiguous(), up_biases.contiguous()
     L = _lib.lib()
-    need = _qmv_workspace(L, m, k, n, group_size, bits, 2)
-    ws = workspace(values.device, need) if need else None
+    ws = _qmv_workspace(L, values.device, m, k, n, group_size, bits, 2)
     fn = L.mt_affine_swiglu_repacked if _repacked(gw) else L.mt_affine_swiglu
     _lib.check(fn(
         x.data_ptr(), gw.data_ptr(), gs.data_ptr(), gb.data_ptr(), uw.data_ptr(), us.data_ptr(),
         ub.data_ptr(), out.data_ptr(), m, k, n, group_size, bits, code, _ptr(ws),
         0 if ws is None else ws.numel(), _stream_handle(values.device)))
     return out
+
+
+def _mlp_workspace(L, device, need, m, hdim, idim, group_size, bits, stream=None):
+    """The workspace of an MLP call, ``need`` being its rows query's answer."""
+    if m <= _dispatch_rows(group_size) or not need:  # 0: a shape that the call will refuse
+        return workspace(device, need, stream)
+    return _many_rows_workspace(
+        device, need, lambda: L.mt_affine_mlp_workspace_bytes(m, hdim, idim, group_size, bits),
+        stream)
 
 
 def affine_mlp(values, gate, up, down, *, group_size=64, bits=4, residual=None):
@@ -263,8 +288,9 @@ def affine_mlp(values, gate, up, down, *, group_size=64, bits=4, residual=None):
     tensors = [_as_u32(gw), gs.contiguous(), gb.contiguous(), _as_u32(uw), us.contiguous(),
                ub.contiguous(), _as_u32(dw), ds.contiguous(), db.contiguous()]
     L = _lib.lib()
-    need = L.mt_affine_mlp_rows_workspace_bytes(m, hdim, idim, group_size, bits)
-    ws = workspace(values.device, need)
+    ws = _mlp_workspace(
+        L, values.device, L.mt_affine_mlp_rows_workspace_bytes(m, hdim, idim, group_size, bits),
+        m, hdim, idim, group_size, bits)
     args = (x.data_ptr(), *[t.data_ptr() for t in tensors], _ptr(res), out.data_ptr(), m, hdim,
             idim, group_size, bits, code)
     tail = (ws.data_ptr(), ws.numel(), _stream_handle(values.device))
@@ -346,7 +372,8 @@ class BoundMlp:
             if need is None:  # installed plans may change the need: refreshed on a refusal
                 need = self.need[m] = L.mt_affine_mlp_rows_workspace_bytes(
                     m, self.hdim, self.idim, self.group_size, self.bits)
-            ws = workspace(self.device, need, stream)
+            ws = _mlp_workspace(L, self.device, need, m, self.hdim, self.idim, self.group_size,
+                                self.bits, stream)
             st = L.mt_affine_mlp_layouts(
                 x.data_ptr(), *self.wptrs, rptr, out.data_ptr(), m, self.hdim, self.idim,
                 self.group_size, self.bits, self.code, *self.layouts, ws.data_ptr(), ws.numel(),
@@ -425,9 +452,9 @@ def affine_matmul(values, weight, scales, biases, *, group_size=64, bits=4):
     w = _as_u32(weight)
     s, b = scales.contiguous(), biases.contiguous()
     lib = _lib.lib()
-    need = max(lib.mt_affine_gemm_workspace_bytes(m, k, n, group_size, bits),
-               lib.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, 1))
-    ws = workspace(values.device, need) if need else None
+    need = lib.mt_affine_gemm_workspace_bytes(m, k, n, group_size, bits)
+    wide = lib.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, 1)
+    ws = _many_rows_workspace(values.device, max(need, wide), lambda: need)
     _lib.check(lib.mt_affine_gemm(
         x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), out.data_ptr(), m, k, n,
         group_size, bits, code, _ptr(ws), 0 if ws is None else ws.numel(),
@@ -676,7 +703,7 @@ def bind_mlp_executor(sample_values, mlx, packed, sample_residual, *, group_size
         (down_weight, down_scales, down_biases) = mlx
     chosen = {}  # row bucket -> (gate, up, down) in the layouts picked for it
 
-    chunk = 16 if group_size == 32 else 32  # rows of one dispatch
+    chunk = _dispatch_rows(group_size)
 
     def bucket(values):
         rows = values.numel() // values.shape[-1]

@@ -239,3 +239,67 @@ def test_residual_and_output_at_an_odd_element(dtype, repacked):
                                 ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
     assert torch.equal(bits(buf[1:1 + m * n].view(m, n)), bits(want))
     assert float(buf[0]) == 7.0 and bool((buf[1 + m * n:] == 7.0).all())
+
+
+def _captured(call, warm, monkeypatch):
+    """Replays of ``call`` captured on a stream whose only workspace is that of ``warm``."""
+    from metile_amd import quantized
+
+    monkeypatch.setattr(quantized, "_workspaces", {})
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    if warm is not None:
+        with torch.cuda.stream(side):
+            warm()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = call()
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        yield out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,warm", [(64, 4864, 896, 8),   # K split, a buffer for the row dispatches
+                                        (40, 1536, 2048, 0)])  # row dispatches need none at all
+def test_capture_with_the_workspace_of_the_row_dispatches(m, k, n, warm, monkeypatch):
+    """Inside capture a workspace cannot grow: a call whose row dispatches have room runs as them."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    lib = _lib.lib()
+    least = lib.mt_affine_qmv_workspace_bytes(m, k, n, 64, 4, 1)
+    assert least <= (1 << 20 if warm else 0) < lib.mt_affine_rows_workspace_bytes(m, k, n, 64, 4, 1)
+    w = affine_to_torch(O.make_affine_weight(n, k, 4, 64, 56, 10), "bf16")
+    x = act_to_torch(O.make_activations(m, k, 56), "bf16")
+    want = torch.cat([mt.affine_qmv(x[:32], *w), mt.affine_qmv(x[32:], *w)])
+    for out in _captured(lambda: mt.affine_qmv(x, *w),
+                         (lambda: mt.affine_qmv(x[:warm], *w)) if warm else None, monkeypatch):
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bound", [False, True])
+def test_mlp_capture_with_the_workspace_of_the_row_dispatches(bound, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    h, i, m = 512, 4096, 48
+    lib = _lib.lib()
+    assert (lib.mt_affine_mlp_workspace_bytes(m, h, i, 64, 4) <= 1 << 20
+            < lib.mt_affine_mlp_rows_workspace_bytes(m, h, i, 64, 4))
+    weights = [affine_to_torch(O.make_affine_weight(n, k, 4, 64, 57, 10 + 2 * p), "bf16")
+               for p, (n, k) in enumerate(((i, h), (i, h), (h, i)))]
+    x = act_to_torch(O.make_activations(m, h, 57), "bf16")
+    call = mt.quantized.BoundMlp(*weights) if bound else (lambda v: mt.affine_mlp(v, *weights))
+    ws = torch.zeros(lib.mt_affine_mlp_workspace_bytes(m, h, i, 64, 4), dtype=torch.uint8,
+                     device="cuda")
+    want = torch.empty_like(x)
+    _lib.check(lib.mt_affine_mlp(
+        x.data_ptr(), *(t.data_ptr() for triple in weights for t in triple), None, want.data_ptr(),
+        m, h, i, 64, 4, _lib.MT_BF16, ws.data_ptr(), ws.numel(),
+        torch.cuda.current_stream().cuda_stream))
+    for out in _captured(lambda: call(x), lambda: call(x[:8]), monkeypatch):
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
