@@ -58,8 +58,9 @@ size_t mt_affine_qmv_workspace_bytes(int M, int K, int N, int group_size, int bi
  * Replaces mlx_affine_qmv (metile/backends/mlx_quantized.py:691-714) and, with a residual,
  * mlx_affine_residual_qmv (metile/backends/mlx_quantized.py:1538-1624); the kernels they
  * bind are kernels/affine_qmv.py:57-132. bits in {4, 8}; group_size a power of two >= 32
- * that divides K; K % 64 == 0; N % 32 == 0; any M >= 1 (rows beyond 32 run in 32-row
- * chunks, 16-row chunks for groups of 32). */
+ * that divides K; K % 64 == 0; N % 32 == 0; any M >= 1 (more than 32 rows, 16 for groups of
+ * 32, run as one launch of the wide kernel or in chunks of that many: see
+ * mt_affine_rows_workspace_bytes). */
 int mt_affine_qmv(const void* x, const uint32_t* w_q, const void* scales, const void* biases,
                   const void* residual, void* y, int M, int K, int N, int group_size, int bits,
                   int dtype, void* workspace, size_t workspace_bytes, void* stream);
@@ -289,8 +290,8 @@ typedef struct mt_gemm_plan {
  * metile/backends/mlx_affine.py:36-41 with _candidate_configs :157-166). Host-only: they touch
  * no device.
  *
- * M is the rows of one dispatch (1..32, 1..16 for groups of 32; calls with more rows run
- * dispatches of that many); nproj 1 (QMV) or 2 (SwiGLU).
+ * M is the rows of one dispatch (1..32, 1..16 for groups of 32; calls with more rows run the wide
+ * kernel, mt_affine_rows_plan, or dispatches of that many); nproj 1 (QMV) or 2 (SwiGLU).
  * Within an MLP call, the gate/up dispatch is the nproj = 2 shape (K = H, N = I) and the down
  * dispatch the nproj = 1 shape (K = I, N = H). */
 
@@ -304,6 +305,17 @@ int mt_affine_qmv_plan_candidates(int M, int K, int N, int group_size, int bits,
 /* Install `plan` for the shape (rejects a plan the kernels cannot run); NULL removes it. */
 int mt_affine_qmv_plan_set(int M, int K, int N, int group_size, int bits, int nproj, int dtype,
                            const mt_qmv_plan* plan);
+/* How a QMV or SwiGLU call of any M rows runs, given the workspace of mt_affine_rows_workspace_bytes:
+ * the wide kernel's tile (rows, columns) and K splits, or zeros where it runs as row dispatches (32
+ * rows at a time, 16 for groups of 32), each with the plan above. The wide kernel plans itself:
+ * installed QMV plans are plans of dispatches and do not change it. */
+typedef struct mt_rows_plan {
+  int tile_m;
+  int tile_n;
+  int ksplit;
+} mt_rows_plan;
+int mt_affine_rows_plan(int M, int K, int N, int group_size, int bits, int nproj, int dtype,
+                        mt_rows_plan* out);
 /* The same three for the prefill GEMM (4-bit; M = rows of the call, bucketed likewise). With no plan
  * installed the first gives the planner's, which runs where the wide kernel does not. */
 int mt_affine_gemm_plan(int M, int K, int N, int group_size, int dtype, mt_gemm_plan* out);

@@ -38,6 +38,12 @@ class QmvPlan(ctypes.Structure):
                 ("tiles", ctypes.c_int), ("order", ctypes.c_int)]
 
 
+class RowsPlan(ctypes.Structure):
+    """``mt_rows_plan``."""
+
+    _fields_ = [("tile_m", ctypes.c_int), ("tile_n", ctypes.c_int), ("ksplit", ctypes.c_int)]
+
+
 class GemmPlan(ctypes.Structure):
     """``mt_gemm_plan``."""
 
@@ -55,6 +61,7 @@ _P = ctypes.c_void_p
 _I = ctypes.c_int
 _Z = ctypes.c_size_t
 _QP = ctypes.POINTER(QmvPlan)
+_RP = ctypes.POINTER(RowsPlan)
 _GP = ctypes.POINTER(GemmPlan)
 _DP = ctypes.POINTER(DensePlan)
 
@@ -93,6 +100,7 @@ SIGNATURES = {
     "mt_affine_qmv_plan": (_I, [_I, _I, _I, _I, _I, _I, _I, _QP]),
     "mt_affine_qmv_plan_candidates": (_I, [_I, _I, _I, _I, _I, _I, _QP, _I]),
     "mt_affine_qmv_plan_set": (_I, [_I, _I, _I, _I, _I, _I, _I, _QP]),
+    "mt_affine_rows_plan": (_I, [_I, _I, _I, _I, _I, _I, _I, _RP]),
     "mt_affine_gemm_plan": (_I, [_I, _I, _I, _I, _I, _GP]),
     "mt_affine_gemm_plan_candidates": (_I, [_I, _I, _I, _I, _GP, _I]),
     "mt_affine_gemm_plan_set": (_I, [_I, _I, _I, _I, _I, _GP]),

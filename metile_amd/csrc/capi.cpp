@@ -798,6 +798,15 @@ bool use_wide(int M, int K, int N, int nproj, int group_size, int bits, const vo
   return need == 0 || (workspace && workspace_bytes >= need);
 }
 
+// Whether a QMV or SwiGLU call of this shape is one for the wide kernel: more rows than one dispatch
+// takes, and none that its dispatches would refuse (groups of 32 that no staged plan fits).
+bool many_rows(int M, int K, int N, int nproj, int group_size, int bits, int dtype) {
+  const int chunk = row_chunk(group_size);
+  return M > chunk &&
+         (group_size != 32 ||
+          plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER);
+}
+
 int run_wide(const char* op, const WidePlan& plan, int nproj, const void* x,
              const uint32_t* const w[2], const void* const s[2], const void* const b[2],
              const void* residual, void* y, int M, int K, int N, int group_size, int bits, int dtype,
@@ -848,12 +857,9 @@ int run_qmv(const char* op, int nproj, const void* x, const uint32_t* const w[2]
   if (need && (!workspace || workspace_bytes < need))
     return fail(MT_ERR_WORKSPACE, std::string(op) + ": workspace of " + std::to_string(need) +
                                       " bytes required, got " + std::to_string(workspace_bytes));
-  // A call that the row chunks would refuse is refused: the workspace above, and below a group of 32
-  // that no staged plan fits.
+  // A call that the row chunks would refuse is refused (its workspace above, its plan below).
   WidePlan wide;
-  if (M > chunk && wide_aligned(x, residual, y) &&
-      (group_size != 32 ||
-       plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER) &&
+  if (many_rows(M, K, N, nproj, group_size, bits, dtype) && wide_aligned(x, residual, y) &&
       use_wide(M, K, N, nproj, group_size, bits, workspace, workspace_bytes, &wide))
     return run_wide(op, wide, nproj, x, w, s, b, residual, y, M, K, N, group_size, bits, dtype,
                     workspace, stream, layout);
@@ -1439,6 +1445,20 @@ size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int b
   WidePlan w;
   if (M <= row_chunk(group_size) || !plan_wide(M, K, N, np, group_size, bits, &w)) return 0;
   return std::max(wide_bytes(w), qmv_workspace(M, K, N, np, group_size, bits));
+}
+
+int mt_affine_rows_plan(int M, int K, int N, int group_size, int bits, int nproj, int dtype,
+                        mt_rows_plan* out) {
+  const int st = check_affine("mt_affine_rows_plan", M, K, N, group_size, bits, dtype);
+  if (st) return st;
+  if (!out) return fail(MT_ERR_INVALID_ARGUMENT, "mt_affine_rows_plan: null output");
+  const int np = nproj == 2 ? 2 : 1;
+  WidePlan w{};
+  if (!many_rows(M, K, N, np, group_size, bits, dtype) ||
+      !plan_wide(M, K, N, np, group_size, bits, &w))
+    w = WidePlan{};
+  *out = mt_rows_plan{w.tile_m, w.tile_n, w.ksplit};
+  return MT_OK;
 }
 
 size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits) {

@@ -703,11 +703,8 @@ def bind_mlp_executor(sample_values, mlx, packed, sample_residual, *, group_size
         (down_weight, down_scales, down_biases) = mlx
     chosen = {}  # row bucket -> (gate, up, down) in the layouts picked for it
 
-    chunk = _dispatch_rows(group_size)
-
-    def bucket(values):
-        rows = values.numel() // values.shape[-1]
-        return _tuning.row_bucket(min(max(rows, 1), chunk))
+    def bucket(values):  # beyond the chunk the wide kernel's, whose layouts are decided apart
+        return _tuning.row_bucket(max(values.numel() // values.shape[-1], 1))
 
     def stages(values):
         key = bucket(values)

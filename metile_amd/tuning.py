@@ -265,6 +265,22 @@ def install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, plan) -> None:
                                                  _dtype_code(dtype), c))
 
 
+def rows_plan(rows, k, n, group_size, bits, nproj, dtype):
+    """``(tile rows, tile columns, K splits)`` of the wide kernel for a QMV or SwiGLU call of ``rows``
+    rows, or ``None`` where the call runs as row dispatches (each with its ``qmv_plan``)."""
+    out = _lib.RowsPlan()
+    _lib.check(_lib.lib().mt_affine_rows_plan(rows, k, n, group_size, bits, nproj,
+                                              _dtype_code(dtype), ctypes.byref(out)))
+    return (out.tile_m, out.tile_n, out.ksplit) if out.tile_m else None
+
+
+def _wide_call(x, n, group_size, bits, nproj) -> bool:
+    """Whether a call over ``x`` (two-dimensional) runs the wide kernel."""
+    rows, k = x.shape
+    return (rows > (16 if group_size == 32 else 32)
+            and rows_plan(rows, k, n, group_size, bits, nproj, x.dtype) is not None)
+
+
 def gemm_plan(rows, k, n, group_size, dtype) -> GemmPlan:
     out = _lib.GemmPlan()
     _lib.check(_lib.lib().mt_affine_gemm_plan(rows, k, n, group_size, _dtype_code(dtype),
@@ -542,10 +558,11 @@ def _tune_qmv_dispatch(values, weights, group_size, bits, layout):
     return plan, record
 
 
-def _tune_qmv_layouts(values, weight_sets, group_size, bits):
+def _tune_qmv_layouts(values, weight_sets, group_size, bits, wide=False):
     """Measure every plan of one dispatch shape over each ``(layout, weights)`` of
     ``weight_sets`` (the same weights in different code layouts; the first is the baseline's)
-    and return ``(plan or None, layout, record)``: the fastest pair."""
+    and return ``(plan or None, layout, record)``: the fastest pair. ``wide``: a call that runs the
+    wide kernel, which has one plan; only its layouts are measured."""
     from .quantized import _as_u32
 
     L = _lib.lib()
@@ -559,18 +576,24 @@ def _tune_qmv_layouts(values, weight_sets, group_size, bits):
         sets.append((layout, tensors))
     layout0, tensors0 = sets[0]
     n = tensors0[0].shape[1] if layout0 == _LAYOUT_REPACKED else tensors0[0].shape[0]
-    candidates = qmv_plan_candidates(rows, k, n, group_size, bits, nproj)
+    candidates = [] if wide else qmv_plan_candidates(rows, k, n, group_size, bits, nproj)
     copies = _copies(_tensor_bytes(*tensors0))
     rotations = {layout: [tensors] + [[t.clone() for t in tensors] for _ in range(copies - 1)]
                  for layout, tensors in sets}
-    need = 0
+
+    def install(plan):
+        if not wide:
+            install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, plan)
+
+    need = L.mt_affine_rows_workspace_bytes(rows, k, n, group_size, bits, nproj)
     for plan in [None, *candidates]:
-        install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, plan)
+        install(plan)
         need = max(need, L.mt_affine_qmv_workspace_bytes(rows, k, n, group_size, bits, nproj))
-    install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, None)
+    install(None)
     bench = _Bench(values.device, need)
     x = values.contiguous()
-    outs = [torch.empty(rows, n, dtype=dtype, device=values.device) for _ in range(copies)]
+    outs = [torch.empty(rows, n, dtype=dtype, device=values.device)
+            for _ in range(1 if wide else copies)] * (copies if wide else 1)
 
     def body_for(layout):
         fn = ((L.mt_affine_qmv_repacked if layout == _LAYOUT_REPACKED else L.mt_affine_qmv)
@@ -597,26 +620,26 @@ def _tune_qmv_layouts(values, weight_sets, group_size, bits):
         for layout, _ in sets:
             body = body_for(layout)
             for key, plan in [(_BASELINE, None), *[(c, c) for c in candidates]]:
-                install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, plan)
+                install(plan)
                 graphs[(key, layout)] = bench.capture(body)
                 bench.stream.synchronize()
                 if reference is None:
                     reference = outs[0].clone()
                 else:
                     _gate(outs[0], reference, "affine plan tuning")
-        install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, None)
+        install(None)
         # cost: workgroups, then the baseline's layout
         timings, chosen = _tournament(
             bench, graphs, copies,
             lambda key: (-1 if key[0] == _BASELINE else key[0].workgroups, key[1] != layout0),
             baseline)
     finally:
-        install_qmv_plan(rows, k, n, group_size, bits, nproj, dtype, None)
+        install(None)
         bench.close()
-    planner = qmv_plan(rows, k, n, group_size, bits, nproj, dtype)
     plan = None if chosen[0] == _BASELINE else chosen[0]
     record = {
-        "planner": asdict(planner),
+        "planner": (rows_plan(rows, k, n, group_size, bits, nproj, dtype) if wide else
+                    asdict(qmv_plan(rows, k, n, group_size, bits, nproj, dtype))),
         "planner_us": round(timings[baseline] * 1e6, 3),
         "chosen_us": round(timings[chosen] * 1e6, 3),
         "copies": copies,
@@ -648,7 +671,8 @@ def ensure_qmv_plans(values, weights, *, group_size, bits, autotune=True, retune
     (SwiGLU), in MLX or repacked layout (measured in the layout given; the decision applies to
     both). Per dispatch shape: this process's decision, else the disk cache's, else
     (``autotune`` and tuning enabled, outside graph capture) a measurement, which is then
-    cached. Returns ``{rows: plan or None}`` (None: the planner's plan)."""
+    cached. Returns ``{rows: plan or None}`` (None: the planner's plan); empty for a call that runs
+    the wide kernel, which plans itself."""
     from .quantized import _repacked
 
     nproj = len(weights) // 3
@@ -657,6 +681,8 @@ def ensure_qmv_plans(values, weights, *, group_size, bits, autotune=True, retune
     n = weights[0].shape[1] if layout == _LAYOUT_REPACKED else weights[0].shape[0]
     x = values.reshape(-1, k)
     out = {}
+    if _wide_call(x, n, group_size, bits, nproj):
+        return out
     with _lock:
         for rows in dispatch_rows(x.shape[0], group_size):
             mem = ("qmv", values.device.index, row_bucket(rows), k, n, group_size, bits, nproj,
@@ -694,7 +720,8 @@ def ensure_qmv_layout(values, layouts, *, group_size, bits, autotune=True, retun
     the first being the default (its planner plan is the baseline). The first dispatch shape's
     plans are measured over every layout, which picks the plan and the layout together (plans
     are layout-free: results are bit-identical in either layout); the other dispatch shapes are
-    then tuned in that layout. Returns the name of the layout to keep: the first when nothing
+    then tuned in that layout. A call that runs the wide kernel is timed as it is over each layout.
+    Returns the name of the layout to keep: the first when nothing
     was measured (tuning off, or inside graph capture, with no cached decision)."""
     names = list(layouts)
     if not names or any(name not in _LAYOUT_CODES for name in names):
@@ -713,6 +740,8 @@ def ensure_qmv_layout(values, layouts, *, group_size, bits, autotune=True, retun
     k = values.shape[-1]
     n = first[0].shape[1] if names[0] == "repacked" else first[0].shape[0]
     x = values.reshape(-1, k)
+    if _wide_call(x, n, group_size, bits, nproj):
+        return _wide_layout(x, n, layouts, group_size, bits, autotune, retune)
     rows = dispatch_rows(x.shape[0], group_size)[0]
     chosen = names[0]
     with _lock:
@@ -747,6 +776,32 @@ def ensure_qmv_layout(values, layouts, *, group_size, bits, autotune=True, retun
     ensure_qmv_plans(values, layouts[chosen], group_size=group_size, bits=bits,
                      autotune=autotune, retune=False)
     return chosen
+
+
+def _wide_layout(x, n, layouts, group_size, bits, autotune, retune):
+    """``ensure_qmv_layout`` of a call that runs the wide kernel: the layout decided for its rows'
+    bucket (this process's, the disk cache's, or measured now), else the first."""
+    names = list(layouts)
+    nproj = len(layouts[names[0]]) // 3
+    rows, k = x.shape
+    lmem = ("wide", x.device.index, row_bucket(rows), k, n, group_size, bits, nproj, x.dtype,
+            tuple(names))
+    with _lock:
+        if lmem in _decided_layouts and not retune:
+            return _decided_layouts[lmem][1]
+        shape = {**_qmv_shape(rows, k, n, group_size, bits, nproj, x.dtype), "layouts": names}
+        key = _persistent_key(x.device, "affine_wide_layout", shape, [])
+        found, _, chosen = (False, None, None) if retune else _read_layout_decision(key)
+        if not found or chosen not in names:
+            if not autotune or not tuning_enabled() or torch.cuda.is_current_stream_capturing():
+                return names[0]
+            _, code, record = _tune_qmv_layouts(
+                x, [(_LAYOUT_CODES[name], layouts[name]) for name in names], group_size, bits,
+                wide=True)
+            chosen = _LAYOUT_NAMES[code]
+            _write_decision(key, None, {"op": "affine_wide_layout", **shape, **record})
+        _decided_layouts[lmem] = (None, chosen)
+        return chosen
 
 
 def _read_layout_decision(key):
@@ -940,7 +995,10 @@ def dispatches(op: str) -> tuple:
     Each dict holds the shape (``rows`` is the row bucket the decision covers), the plan the
     library runs for it now, the code layout when a layout decision picked one, and
     ``source``: ``"measured"``, ``"cached"`` (from the decision cache on disk) or ``"planner"``
-    (nothing decided; the library's own plan)."""
+    (nothing decided; the library's own plan). QMV and SwiGLU calls of more rows than one dispatch
+    run the wide kernel, which has no plan to decide (``rows_plan`` tells how), and are not listed;
+    a matmul record's ``wide`` says that its calls run that kernel, for which no plan beat it, and
+    that the plan named runs only where its workspace is not given."""
     if op not in ("swiglu", "qmv", "matmul"):
         raise ValueError('op must be "swiglu", "qmv" or "matmul"')
     with _lock:
@@ -959,6 +1017,8 @@ def dispatches(op: str) -> tuple:
                         "dtype": str(dtype), "group_size": group_size, "bits": 4,
                         "device": device, "kernel": plan.kernel, "tile_m": plan.tile_m,
                         "tile_n": plan.tile_n, "ksplit": plan.ksplit, "order": plan.order,
+                        "wide": decided.get(mem) is None and rows_plan(
+                            bucket, k, n, group_size, 4, 1, dtype) is not None,
                         "source": source})
             continue
         if mem[0] != "qmv" or mem[7] != (2 if op == "swiglu" else 1):

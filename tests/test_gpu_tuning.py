@@ -229,6 +229,31 @@ def test_layout_decision_persists_and_reloads(monkeypatch, tmp_path):
     assert tuning.qmv_plan(1, 8960, 1536, 64, 4, 1, torch.bfloat16) == installed
 
 
+def test_executor_times_calls_of_the_wide_kernel_themselves(monkeypatch, tmp_path):
+    # 40 rows: each stage's layout from the call as it runs, no plans of 32- and 8-row dispatches;
+    # a three-row call then decides its own
+    monkeypatch.setenv("METILE_AMD_CACHE_DIR", str(tmp_path))
+    monkeypatch.delenv("METILE_AMD_DISABLE_TUNING", raising=False)
+    gate = O.make_affine_weight(4864, 896, 4, 64, 5, 10)
+    up = O.make_affine_weight(4864, 896, 4, 64, 5, 12)
+    down = O.make_affine_weight(896, 4864, 4, 64, 5, 14)
+    x = O.make_activations(40, 896, 5)
+    res = O.make_activations(40, 896, 5, tensor_id=3)
+    xt, rt = act_to_torch(x, "bf16"), act_to_torch(res, "bf16")
+    ts = [affine_to_torch(w, "bf16") for w in (gate, up, down)]
+    ex = mt.mlx_affine_mlp_executor(xt, *ts[0], *ts[1], *ts[2], rt)
+    entries = list(tuning.load_decisions().values())
+    assert [(e["op"], e["rows"]) for e in entries] == [("affine_wide_layout", 64)] * 2
+    print(f"[tuner wide 40 rows] {[(e['layout'], e['planner_us'], e['chosen_us']) for e in entries]}",
+          flush=True)
+    for m in (40, 3):
+        ref, _ = O.affine_mlp(x[:m], gate, up, down, 64, 4, residual=res[:m])
+        _check(f"executor, {m} rows", torch_to_act(ex(xt[:m], rt[:m]), "bf16"), ref,
+               min_exact=0.85)
+    assert {(e["op"], e["rows"]) for e in tuning.load_decisions().values()} == {
+        ("affine_wide_layout", 64), ("affine_qmv_layout", 4)}
+
+
 def test_tuned_executor_and_gemm(monkeypatch, tmp_path):
     monkeypatch.setenv("METILE_AMD_CACHE_DIR", str(tmp_path))
     monkeypatch.delenv("METILE_AMD_DISABLE_TUNING", raising=False)

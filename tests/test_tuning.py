@@ -547,6 +547,65 @@ def test_dispatches_report_the_plan_of_the_dispatch_rows_not_the_bucket(clean_pl
     assert got == tuning.qmv_plan(3, k, n, 64, 4, 2, bf)
 
 
+def _weights(n, k, g, bits, nproj):
+    one = (torch.zeros(n, k * bits // 32, dtype=torch.int32),
+           torch.zeros(n, k // g, dtype=torch.bfloat16), torch.zeros(n, k // g, dtype=torch.bfloat16))
+    return one * nproj
+
+
+@pytest.mark.parametrize("rows,bits,g,wide", [
+    (32, 4, 64, False), (33, 4, 64, True), (333, 4, 128, True), (33, 8, 64, True),
+    (16, 8, 32, False), (17, 8, 32, True), (48, 4, 32, False)])
+def test_calls_of_the_wide_kernel_measure_no_row_plans(rows, bits, g, wide, clean_plans, monkeypatch,
+                                                       tmp_path):
+    """A call runs the wide kernel or row dispatches; the tuner measures what the call runs: no
+    plans of dispatches that it does not make, and its layout on the call itself."""
+    monkeypatch.setenv("METILE_AMD_CACHE_DIR", str(tmp_path))
+    monkeypatch.delenv("METILE_AMD_DISABLE_TUNING", raising=False)
+    monkeypatch.setattr(tuning, "_device_identity", lambda device: {"architecture": "cpu-test"})
+    measured = []
+
+    def layouts(values, sets, group_size, bits, wide=False):
+        measured.append((values.shape[0], [layout for layout, _ in sets], wide))
+        return None, sets[-1][0], {"layout": "mlx"}
+
+    monkeypatch.setattr(tuning, "_tune_qmv_layouts", layouts)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    k, n = 512, 256
+    x = torch.zeros(rows, k, dtype=torch.bfloat16)
+    mlx = _weights(n, k, g, bits, 2)
+    assert (tuning.rows_plan(rows, k, n, g, bits, 2, x.dtype) is not None) == wide
+    decided = tuning.ensure_qmv_plans(x, mlx, group_size=g, bits=bits)
+    chunk = 16 if g == 32 else 32
+    if wide:
+        assert decided == {} and measured == [] and tuning.dispatches("swiglu") == ()
+    else:
+        assert [m[0] for m in measured] == [min(rows, chunk)] and len(decided) == 1
+    measured.clear()
+    packed = tuple(torch.zeros(k // 64, n, 2 * bits, dtype=torch.int32) if i % 3 == 0 else t
+                   for i, t in enumerate(mlx))
+    for _ in range(2):  # decided once
+        assert tuning.ensure_qmv_layout(x, {"repacked": packed, "mlx": mlx}, group_size=g,
+                                        bits=bits) == "mlx"
+    assert measured == [(rows if wide else min(rows, chunk), [1, 0], wide)]
+    tuning.clear_plans()  # a fresh process state: the layout comes back from the log
+    measured.clear()
+    assert tuning.ensure_qmv_layout(x, {"repacked": packed, "mlx": mlx}, group_size=g,
+                                    bits=bits) == "mlx"
+    assert measured == []
+
+
+def test_matmul_records_say_where_the_wide_kernel_runs(clean_plans):
+    bf = torch.bfloat16
+    for rows, plan in ((512, None), (256, GemmPlan("ring", 128, 96, 1)), (32, None)):
+        mem = ("gemm", 0, rows, 1536, 8960, 64, bf)
+        with tuning._lock:
+            tuning._resolved[mem] = "measured"
+            tuning._decided[mem] = plan
+    assert {d["rows"]: d["wide"] for d in tuning.dispatches("matmul")} == {
+        512: True, 256: False, 32: False}
+
+
 def test_gemv4_plans_are_checked(clean_plans):
     import torch
 
