@@ -81,8 +81,9 @@ size_t mt_affine_mlp_workspace_bytes(int M, int H, int I, int group_size, int bi
  * of the wide kernel, which reads the weights once per row tile of up to 128 rows, where the format
  * allows (4-bit groups of 64 or more, 8-bit groups of 32 or more; x and y below 2 GiB) and the
  * workspace holds its split-K partials: at least these many bytes. With less they run as row
- * dispatches within the sizes of the queries above. Both cover the sizes of the queries above too
- * (the first is 0 where the wide kernel does not apply). No
+ * dispatches within the sizes of the queries above: results then differ in the order of the fp32
+ * sums. Both cover the sizes of the queries above too (the first is 0 where the wide kernel does not
+ * apply). Neither grows with M: a workspace for several M takes the largest of their sizes. No
  * counterpart in the reference, whose row kernels loop. */
 size_t mt_affine_rows_workspace_bytes(int M, int K, int N, int group_size, int bits, int nproj);
 size_t mt_affine_mlp_rows_workspace_bytes(int M, int H, int I, int group_size, int bits);
@@ -103,10 +104,13 @@ int mt_affine_mlp(const void* x, const uint32_t* gate_w, const void* gate_scales
  * counterpart in the reference. The workspace lives in a 16 MiB device array inside the library
  * (one per GPU, held until the process ends); a call whose mt_affine_mlp_workspace_bytes exceeds
  * 16 MiB fails with MT_ERR_WORKSPACE. It allocates nothing (no hipMalloc, no allocating library
- * call); the first call on a device clears the array's counter region with a small kernel on
- * `stream`. Every call on a GPU shares that array: calls that overlap on one GPU (other
+ * call); the array's counter region is zero when the library is loaded and after every call. Every
+ * call on a GPU shares that array: calls that overlap on one GPU (other
  * streams, or a graph captured over this call replayed while another runs) race. Same arguments
- * (minus the workspace) and results as mt_affine_mlp, bit for bit. */
+ * (minus the workspace) and results as mt_affine_mlp given a 16 MiB workspace, bit for bit: up to 32
+ * rows (16 for groups of 32) those of every sufficient workspace; with more rows the wide kernel runs
+ * where mt_affine_mlp_rows_workspace_bytes is at most 16 MiB, else only in a stage whose K it need
+ * not split. */
 int mt_affine_mlp_noalloc(const void* x, const uint32_t* gate_w, const void* gate_scales,
                           const void* gate_biases, const uint32_t* up_w, const void* up_scales,
                           const void* up_biases, const uint32_t* down_w, const void* down_scales,

@@ -13,12 +13,13 @@ from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
 from metile_amd import _lib
 from oracle import affine as O
-from tests.helpers import act_to_torch, affine_to_torch
+from tests.helpers import act_to_torch, affine_to_torch, torch_to_act
 
 H, I, G, BITS = 1536, 8960, 64, 4
 
@@ -117,3 +118,41 @@ def test_noalloc_matches_mt_affine_mlp_on_two_calls_second_smaller():
         torch.cuda.synchronize()
         assert torch.cuda.mem_get_info()[0] == free_before, "the call allocated device memory"
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,wide", [(48, True), (330, False)])
+def test_noalloc_runs_what_a_16_mib_workspace_allows(m, wide):
+    """More rows than one dispatch: the bits of mt_affine_mlp with 16 MiB, where the wide kernel's
+    partial sums fit and where they do not (with a larger workspace the sums' order is another)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    lib = _lib.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    rows_need = lib.mt_affine_mlp_rows_workspace_bytes(m, H, I, G, BITS)
+    assert lib.mt_affine_mlp_workspace_bytes(m, H, I, G, BITS) <= 16 << 20
+    assert (rows_need <= 16 << 20) == wide
+    ptrs, keep = _weights()
+    x = act_to_torch(O.make_activations(m, H, 32), "bf16")
+    r = act_to_torch(O.make_activations(m, H, 32, tensor_id=3), "bf16")
+
+    def with_workspace(nbytes):
+        out = torch.empty_like(x)
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.mt_affine_mlp(x.data_ptr(), *ptrs, r.data_ptr(), out.data_ptr(), m, H, I, G,
+                                     BITS, _lib.MT_BF16, ws.data_ptr(), ws.numel(), stream))
+        torch.cuda.synchronize()
+        return out
+
+    got = torch.empty_like(x)
+    _lib.check(lib.mt_affine_mlp_noalloc(x.data_ptr(), *ptrs, r.data_ptr(), got.data_ptr(), m, H, I,
+                                         G, BITS, _lib.MT_BF16, stream))
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), with_workspace(16 << 20).view(torch.int16))
+    weights = [O.make_affine_weight(n, k, BITS, G, 31, t)
+               for n, k, t in ((I, H, 10), (I, H, 12), (H, I, 14))]
+    ref, _ = O.affine_mlp(O.make_activations(m, H, 32), *weights, G, BITS,
+                          residual=O.make_activations(m, H, 32, tensor_id=3), acc=np.float32)
+    for out in (got, with_workspace(max(rows_need, 16 << 20))):
+        err = O.tolerance_error(torch_to_act(out, "bf16"), ref)
+        assert err <= 2e-3, err
