@@ -930,19 +930,18 @@ constexpr int kDenseRowChunk = 128;  // rows per dense dispatch
 constexpr int kDenseSubChunk = 64;
 
 // Rows per chunk of a dispatch, 0 for one chunk. One chunk has the weights delivered once, two bring
-// them to twice as many CUs from one L2. Two projections are chunked where one chunk would leave a
-// quarter of the CUs idle or a second round mostly empty (at 100 rows 2048 -> 5632, 176 strips, 20.2
-// -> 16.2 us, and 1536 -> 8960, 280 strips, 26.9 -> 22.5; not 2048 -> 8192, 256 strips, 20.4 against
-// 20.7, nor 4096 -> 14336, 68.7 against 77.2); one projection up to 64 MiB of weights, which stay in
-// the caches (8192 -> 2048 19.5 -> 16.3, 8192 -> 3072, 50 MB, 34.6 -> 26.6; not 14336 -> 4096,
-// 117 MB, 46.7 against 53.9).
+// them to twice as many CUs from one L2. Two projections are chunked where both chunks fit side by side,
+// a workgroup a CU (us with weights from memory, two chunks against one, 100 rows: 1024 -> 3072, 96
+// strips, 9.7 against 11.6, 1024 -> 4096, 128 strips, 9.9 against 11.7; not 896 -> 4864, 152 strips, 14.1
+// against 10.9, nor 2048 -> 5632, 176 strips, 22.8 against 19.4, 1536 -> 8960, 280 strips, 27.1 against
+// 25.7; with the weights in the caches two chunks are the faster ones up to 12% there, which a model of
+// many layers does not see). One projection: up to 64 MiB of weights (8960 -> 1536 17.5 against 15.9, in
+// the caches 14.3 against 16.0; 4864 -> 896 10.5 against 11.9; not 14336 -> 4096, 117 MB, 52.6 against
+// 45.0).
 int dense_row_chunk(int rows, int K, int N, int nproj, int ksplit) {
   if (rows <= kDenseSubChunk) return 0;
   if (nproj == 1) return (size_t)K * N * 2 <= (64u << 20) ? kDenseSubChunk : 0;
-  const int cus = device_cus();
-  const long tiles = (long)(N / 32) * ksplit;
-  const bool idle = tiles * 4 < cus * 3L, tail = tiles > cus && tiles * 4 <= cus * 5L;
-  return idle || tail ? kDenseSubChunk : 0;
+  return 2L * (N / 32) * ksplit <= device_cus() ? kDenseSubChunk : 0;
 }
 
 // Dense plans: the K split of every dispatch of a (K, N) shape. Keyed without the rows, so that
@@ -1053,6 +1052,7 @@ int run_dense(const char* op, int nproj, const void* x, const void* const w[2],
     p.ksplit = plan.ksplit;
     p.steps_per_split = plan.steps_per_split;
     p.row_chunk = dense_row_chunk(rows, K, N, nproj, plan.ksplit);
+    p.reread = M - r0 > rows;
     const hipError_t e = mt::launch_dense_qmv(p, dtype, nproj, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, op);
   }

@@ -16,8 +16,9 @@ struct DenseParams {
   int M, K, N;
   int ksplit;
   int steps_per_split;
-  int row_chunk;             // 64: rows per grid z index (rows [z row_chunk, ...) of this launch,
-                             // each with its own partials and counters); 0: one chunk of M rows
+  int reread;                // a later launch of the call reads the weights again
+  int row_chunk;             // 64: rows of a chunk (rows [64 c, ...) of this launch), each with its
+                             // own partials and counters; 0: one chunk of M rows
 };
 
 hipError_t launch_dense_qmv(const DenseParams& p, int dtype, int nproj, hipStream_t stream);

@@ -303,11 +303,14 @@ __global__ __launch_bounds__(kThreads, 2) void dense_qmv_kernel(const DenseParam
 //
 // What bounds it: 2048 -> 8192 runs at the weights' rate from memory, more strips and rows at
 // what a CU receives (about 20 bytes a clock, activations and weights together; a ring of six steps
-// instead of three, or reading operands a step ahead, changed nothing). Measured (MI355X, bf16, gate
-// and up / down; before: K quarter a wave, over 64 rows in two chunks): 2048 -> 8192 at 64 rows 18.5
-// / 15.3 -> 17.1 / 14.8 us, at 128 22.1 / 21.0 -> 21.0 / 16.5; 4096 -> 14336 at 100 rows 93.3 / 54.3
-// -> 68.7 / 46.7; 5120 -> 17408 at 100 rows 174.5 / 86.8 -> 111 / 81.
-// NT: weights read once, with the non-temporal hint; not where a second row chunk reads them again.
+// instead of three, or reading operands a step ahead, changed nothing). Measured (MI355X, bf16, weights
+// from memory, gate and up / down, us; before: K quarter a wave, over 64 rows in two chunks): 2048 ->
+// 8192 at 64 rows 18.5 / 14.3 -> 18.3 / 14.0 (at 33 rows 16.6 / 12.6 -> 17.9 / 12.5: the one size where
+// the kernel before was faster), at 128 26.5 / 21.4 -> 21.4 / 20.9; 4096 -> 14336 at 100 rows 102 / 55 ->
+// 70 / 45; 5120 -> 17408 at 100 rows 181 / 88 -> 110 / 78.
+// NT: weights read once, with the non-temporal hint; not where a second row chunk or a later launch of
+// the call reads them again (5120 -> 17408 at 160 rows, 128 and 32, with the hint 201 / 133, without 186 /
+// 125 us).
 template <int DT, int MT, int NPROJ, int D, bool NT>
 __global__ __launch_bounds__(kThreads, 2) void dense_tile_kernel(const DenseParams args) {
   const DenseParams p = preload_args(args);
@@ -331,17 +334,26 @@ __global__ __launch_bounds__(kThreads, 2) void dense_tile_kernel(const DensePara
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, h = lane >> 5;
   const int K = p.K, N = p.N;
-  // Workgroup -> (row chunk, strip, split). Workgroups go to the 8 XCDs in turn; each takes a
-  // contiguous run with the chunks fastest, so that a strip's chunks meet its weights in one L2.
+  // Workgroup -> (row chunk, strip, split). Workgroups go to the 8 XCDs in turn: strips are dealt out in
+  // that order, a strip's chunks one after the other on its XCD, so that they meet its weights in one L2,
+  // as does a later launch of the call (the kernel above deals strips out alike).
   const int rc = p.row_chunk, chunks = rc ? (p.M + rc - 1) / rc : 1;
   int strip, split, chunk;
   {
-    const int total = gridDim.x, lin = blockIdx.x, k = lin & 7, strips = N / 32;
-    const int item = k * (total >> 3) + min(k, total & 7) + (lin >> 3);
-    const int rest = item / chunks;
-    chunk = item - rest * chunks;
-    split = rest / strips;
-    strip = rest - split * strips;
+    const int lin = blockIdx.x, strips = N / 32, pairs = strips * p.ksplit;  // (strip, split)
+    const int whole = (pairs & ~7) * chunks;  // in groups of 8 pairs; behind them the last few
+    int pair;
+    if (lin < whole) {
+      const int turn = lin >> 3, group = turn / chunks;
+      chunk = turn - group * chunks;
+      pair = 8 * group + (lin & 7);
+    } else {
+      const int left = pairs & 7;
+      chunk = (lin - whole) / left;
+      pair = (pairs & ~7) + (lin - whole) - chunk * left;
+    }
+    split = pair / strips;
+    strip = pair - split * strips;
   }
   const int r0 = chunk * rc;
   const int M = rc ? min(rc, p.M - r0) : p.M;
@@ -645,7 +657,9 @@ hipError_t launch_dense_dt(const DenseParams& p, hipStream_t stream) {
     case 1: return launch_dense_rows<DT, NPROJ>(p, dim3(p.N / 32, p.ksplit), stream);
     case 2: return launch_dense_tile<DT, NPROJ, 2, true>(p, dim3(tiles), stream);
     case 3: return launch_dense_tile<DT, NPROJ, 3, true>(p, dim3(tiles), stream);
-    case 4: return launch_dense_tile<DT, NPROJ, 4, true>(p, dim3(tiles), stream);
+    case 4:  // the only one that others follow
+      return p.reread ? launch_dense_tile<DT, NPROJ, 4, false>(p, dim3(tiles), stream)
+                      : launch_dense_tile<DT, NPROJ, 4, true>(p, dim3(tiles), stream);
   }
   return hipErrorInvalidValue;
 }

@@ -20,6 +20,9 @@ CASES = [
     (1088, 8224, 2, False),    # 257 strips: a second round
     (704, 6112, 2, False),     # 191: a quarter of the CUs idle
     (704, 6144, 2, False),     # 192
+    (704, 4096, 2, False),     # 128: both row chunks at once, a workgroup a CU
+    (704, 4128, 2, False),     # 129: one chunk, strips that 8 does not divide
+    (192, 1024, 2, False),     # two chunks of an even number of strips, empty quarters
     (4160, 320, 1, True),      # K splits of unequal length
     (8192, 2048, 1, True),
     (9216, 4096, 1, True),     # above 64 MiB of weights: one chunk
@@ -95,3 +98,23 @@ def test_residual_and_output_at_an_odd_element(k, n, nproj, dtype):
     got = _run(x, weights, res, buf[1:1 + m * n].view(m, n))
     assert got.data_ptr() % 4 == 2 and torch.equal(got, want)
     assert float(buf[0]) == 7.0 and bool((buf[1 + m * n:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,n,nproj", [(704, 4128, 2), (4160, 320, 1), (192, 1024, 2)])
+def test_rows_beyond_one_launch_equal_single_row_runs(k, n, nproj):
+    """More than 128 rows: launches that others follow (weights read without the hint) and the last
+    one, of one row, of a row kernel's and of a tile's size."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    weights = [(torch.randn(n, k, generator=g, device="cuda") / k**0.5).bfloat16()
+               for _ in range(nproj)]
+    x = torch.randn(300, k, generator=g, device="cuda").bfloat16()
+    rows = (0, 63, 64, 127, 128, 129, 159, 160, 255, 256, 299)
+    alone = {r: _run(x[r:r + 1], weights, None, torch.empty(1, n, dtype=x.dtype, device="cuda"))
+             for r in rows}
+    for m in (129, 160, 200, 256, 300):
+        got = _run(x[:m], weights, None, torch.empty(m, n, dtype=x.dtype, device="cuda"))
+        for r in rows:
+            assert r >= m or torch.equal(got[r], alone[r][0]), (m, r)
