@@ -930,18 +930,22 @@ constexpr int kDenseRowChunk = 128;  // rows per dense dispatch
 constexpr int kDenseSubChunk = 64;
 
 // Rows per chunk of a dispatch, 0 for one chunk. One chunk has the weights delivered once, two bring
-// them to twice as many CUs from one L2. Two projections are chunked where both chunks fit side by side,
-// a workgroup a CU (us with weights from memory, two chunks against one, 100 rows: 1024 -> 3072, 96
-// strips, 9.7 against 11.6, 1024 -> 4096, 128 strips, 9.9 against 11.7; not 896 -> 4864, 152 strips, 14.1
-// against 10.9, nor 2048 -> 5632, 176 strips, 22.8 against 19.4, 1536 -> 8960, 280 strips, 27.1 against
-// 25.7; with the weights in the caches two chunks are the faster ones up to 12% there, which a model of
-// many layers does not see). One projection: up to 64 MiB of weights (8960 -> 1536 17.5 against 15.9, in
-// the caches 14.3 against 16.0; 4864 -> 896 10.5 against 11.9; not 14336 -> 4096, 117 MB, 52.6 against
-// 45.0).
+// them to twice as many CUs from one L2: chunked where both chunks fit side by side, a workgroup a CU,
+// and, from 81 rows with K split, where one chunk would leave a short second round of workgroups. Us with
+// weights from memory, two chunks against one, one projection unless said: gate and up 1024 -> 4096 (128
+// strips) at 100 rows 9.9 against 11.7, 4864 -> 896 10.5 against 11.9; 4864 -> 3072 (288 workgroups) at
+// 128 rows 24.5 against 26.3, 8960 -> 3072 37.1 against 40.4 (at 65 rows 31.2 against 29.0). Not gate and
+// up 896 -> 4864 (152 strips) at 100 rows 14.1 against 10.9, 2048 -> 5632 22.8 against 19.4, 1536 -> 8960
+// 27.1 against 25.7; 8192 -> 2048 (256 workgroups) 18.7 against 17.4, 5120 -> 6144 (384) 36.8 against
+// 33.6. With the weights in the caches two chunks are the faster ones by up to 15% in most of these, which
+// a model of many layers does not see.
 int dense_row_chunk(int rows, int K, int N, int nproj, int ksplit) {
   if (rows <= kDenseSubChunk) return 0;
-  if (nproj == 1) return (size_t)K * N * 2 <= (64u << 20) ? kDenseSubChunk : 0;
-  return 2L * (N / 32) * ksplit <= device_cus() ? kDenseSubChunk : 0;
+  const int cus = device_cus(), wgs = N / 32 * ksplit;
+  if (2 * wgs <= cus) return kDenseSubChunk;
+  const bool tail = ksplit > 1 && K / 64 > 20 * ksplit && wgs > cus && 3 * wgs <= 4 * cus &&
+                    (size_t)nproj * K * N * 2 <= (96u << 20);
+  return tail && rows > 80 ? kDenseSubChunk : 0;
 }
 
 // Dense plans: the K split of every dispatch of a (K, N) shape. Keyed without the rows, so that
@@ -1053,6 +1057,7 @@ int run_dense(const char* op, int nproj, const void* x, const void* const w[2],
     p.steps_per_split = plan.steps_per_split;
     p.row_chunk = dense_row_chunk(rows, K, N, nproj, plan.ksplit);
     p.reread = M - r0 > rows;
+    p.dealt = p.reread && !p.row_chunk && M - r0 - rows <= kRowChunk;
     const hipError_t e = mt::launch_dense_qmv(p, dtype, nproj, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, op);
   }

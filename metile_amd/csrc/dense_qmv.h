@@ -17,6 +17,7 @@ struct DenseParams {
   int ksplit;
   int steps_per_split;
   int reread;                // a later launch of the call reads the weights again
+  int dealt;                 // and it is the row kernel's, which deals its strips out to the XCDs
   int row_chunk;             // 64: rows of a chunk (rows [64 c, ...) of this launch), each with its
                              // own partials and counters; 0: one chunk of M rows
 };
