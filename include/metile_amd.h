@@ -194,8 +194,10 @@ size_t mt_affine_gemm_workspace_bytes(int M, int K, int N, int group_size, int b
  * Dequantization stays exact: the codes enter the MFMAs as exact 16-bit floats (offset + q) and
  * each 64-wide step's partial gets its group's scale and bias terms in fp32. More than 32 rows with
  * no plan installed for the shape take the wide kernel, given its workspace
- * (mt_affine_rows_workspace_bytes); otherwise the installed or the planner's plan below runs.
- * Replaces mlx_affine_matmul / lower_affine_matmul (metile/backends/mlx_affine.py:359-406, metile/compiler/affine_quantized.py:7-99).
+ * (mt_affine_rows_workspace_bytes), unless the planner's plan below is expected to be faster (one round
+ * of tiles that fills the CUs); otherwise the installed or the planner's plan runs. Replaces
+ * mlx_affine_matmul / lower_affine_matmul (metile/backends/mlx_affine.py:359-406,
+ * metile/compiler/affine_quantized.py:7-99).
  * bits = 4; group_size a power of two >= 64 dividing K; K % 64 == 0; N % 32 == 0. */
 int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const void* biases,
                    void* y, int M, int K, int N, int group_size, int bits, int dtype,

@@ -1207,6 +1207,23 @@ GemmPlan planner_gemm(int M, int K, int N) {
   return make_staged(M, K, N, tile, ksplit);
 }
 
+// Whether the ring kernel's plan beats the wide kernel for a call: one round of 128 x 96 tiles that about
+// fills the CUs (512 x 8960 -> 1536 33.9 against 38.4 us, 128 x 3584 -> 6144 20.7 against 24.8). Its time
+// is a fit (rms error 5%) to 391 measured calls of at most one workgroup a CU, the wide kernel's
+// wide_cost, which is 4 to 8% low. Over 785 calls (33 to 2048 rows, K 896 to 18944, N 896 to 18944,
+// groups of 64) it takes 45, which the wide kernel would run 1.057 times as long (worst 1.20, and 0.97
+// where it is wrong); of the others, none has the ring faster by more than 8%, and most are the wide
+// kernel's by far (geometric mean 0.70).
+bool ring_wins(const GemmPlan& g, int M, int K, int N, int group_size, int bits) {
+  WidePlan w;
+  const int cus = device_cus(), wgs = g.tiles * g.ksplit;
+  if (g.kernel != 1 || g.tile_n != 96 || wgs > cus || !plan_wide(M, K, N, 1, group_size, bits, &w))
+    return false;
+  const double ring = 3.9 + 0.637 * g.steps_per_split + (g.ksplit > 1 ? 1.9 + 0.8 * g.ksplit : 0.0) +
+                      2.1 * wgs / cus;
+  return ring < 1.04 * wide_cost(M, K, N, 1, group_size, bits, w);
+}
+
 PlanKey gemm_key(int M, int K, int N, int group_size, int dtype) {
   return PlanKey{kOpGemm, row_bucket(M), K, N, 1, group_size, 4, dtype};
 }
@@ -1648,7 +1665,9 @@ int mt_affine_gemm(const void* x, const uint32_t* w_q, const void* scales, const
   // After the checks: a call of which the plans below would be refused is refused by either kernel.
   mt_gemm_plan installed;
   WidePlan wide;
-  if (M > kRowChunk && wide_aligned(x, nullptr, y) && !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
+  if (M > kRowChunk && wide_aligned(x, nullptr, y) &&
+      !find_gemm_plan(gemm_key(M, K, N, group_size, dtype), &installed) &&
+      !ring_wins(g, M, K, N, group_size, bits) &&
       use_wide(M, K, N, 1, group_size, bits, workspace, workspace_bytes, &wide)) {
     const uint32_t* const w[2] = {w_q, nullptr};
     const void* const s[2] = {scales, nullptr};

@@ -997,8 +997,9 @@ def dispatches(op: str) -> tuple:
     ``source``: ``"measured"``, ``"cached"`` (from the decision cache on disk) or ``"planner"``
     (nothing decided; the library's own plan). QMV and SwiGLU calls of more rows than one dispatch
     run the wide kernel, which has no plan to decide (``rows_plan`` tells how), and are not listed;
-    a matmul record's ``wide`` says that its calls run that kernel, for which no plan beat it, and
-    that the plan named runs only where its workspace is not given."""
+    a matmul record's ``wide`` says that no plan is installed for its calls, which then run that
+    kernel, or the plan named where the library expects that to be faster or the workspace is not
+    given."""
     if op not in ("swiglu", "qmv", "matmul"):
         raise ValueError('op must be "swiglu", "qmv" or "matmul"')
     with _lock:
