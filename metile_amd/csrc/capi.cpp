@@ -799,12 +799,22 @@ bool use_wide(int M, int K, int N, int nproj, int group_size, int bits, const vo
 }
 
 // Whether a QMV or SwiGLU call of this shape is one for the wide kernel: more rows than one dispatch
-// takes, and none that its dispatches would refuse (groups of 32 that no staged plan fits).
+// takes, and none that its dispatches would refuse (groups of 32 that no staged plan fits). Measured
+// against row dispatches just beyond one of them, weights from memory, us as (MLX rows, repacked):
+// 4-bit groups of 64 at 33 rows take 0.67 / 0.78 of the time with one projection, 0.57 / 0.76 with two
+// (geometric means over six MLP shapes; the worst is 2560 -> 6144, 17.7 / 14.2 -> 16.8 / 15.8), 8-bit
+// ones 0.57 / 0.66 and 0.47 / 0.63, groups of 32 at 17 rows 0.66 / 0.74 and 0.58 / 0.65. One projection of
+// short K over groups of 32 keeps two dispatches where the second has one or two rows (the GEMV's): 1536
+// -> 5120 at 17 rows 11.4 / 10.7 against 14.2 / 13.1, 896 -> 3584 8.8 / 8.5 against 10.0 / 9.5; not 2048
+// -> 5120, 15.9 / 15.2 against 14.7 / 13.0.
 bool many_rows(int M, int K, int N, int nproj, int group_size, int bits, int dtype) {
   const int chunk = row_chunk(group_size);
-  return M > chunk &&
-         (group_size != 32 ||
-          plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER);
+  if (M <= chunk) return false;
+  if (group_size == 32 && nproj == 1 && M <= chunk + 2 && K <= 2048 &&
+      N <= (K <= 1536 ? 32 : 16) * device_cus())
+    return false;
+  return group_size != 32 ||
+         plan_qmv(chunk, K, N, nproj, group_size, bits, dtype).kernel != MT_QMV_REGISTER;
 }
 
 int run_wide(const char* op, const WidePlan& plan, int nproj, const void* x,
