@@ -418,25 +418,43 @@ std::string qmv_plan_problem(int rows, int K, int N, int nproj, int group_size, 
   return "";
 }
 
-// Where another kernel than the strip kernels above is the better one in both code layouts (a plan
-// serves both), its plan; else false. Measured over ten (K, N) from 896 x 4864 to 17408 x 5120, cold
-// weights, times against the strip plan's as geometric means (MLX rows, repacked):
+// Where another kernel than the strip kernels above is the better one over both code layouts together
+// (a plan serves both, so that their results stay bit-identical), its plan; else false. Measured over
+// twenty (K, N) from 896 x 4864 to 17408 x 5120, weights from memory, us as (MLX rows, repacked):
 //  * 4-bit codes, one or two rows, K up to 12288 (24 rounds of 512, at most three a wave): the
 //    4x4x4-MFMA GEMV with as many waves as rounds allow and the widest column groups that leave about
 //    two workgroups per CU. Both layouts together take 0.75 / 0.78 of the time with one projection
 //    at one / two rows, 0.76 / 0.78 with two (1536 -> 8960 gate and up at one row 9.5 -> 6.5 and 7.5
 //    -> 6.1 us). Longer K spends more rounds a wave than its loads hide (14336 -> 4096, repacked, at
 //    one row 11.4 -> 14 us).
-//  * 4-bit codes, three or four rows: the same from K = 4096 on, three workgroups for four CUs
+//  * 4-bit codes, three or four rows: the same from K = 4096 on, five workgroups for eight CUs
 //    (4096 -> 14336 gate and up 33.0 -> 20.7 and 21.5 -> 20.0 us, 4864 -> 896 6.0 -> 4.2 and 5.9 ->
 //    4.1 us); below, repacked codes ran up to 1.1 times as long (2048 -> 8192 6.9 -> 7.5 us).
+//    Not from 5120 columns where waves take three rounds (11008 -> 5120 at four rows 18.1 / 13.3 -> 18.1
+//    / 17.2).
+//  * Which column groups: for two projections at one or two rows, or whose waves take several rounds,
+//    two at most (unless eight waves share one round each), the rounds shared evenly: 2560 -> 14336 at
+//    one row with four groups 14.9 / 14.7, with two 12.8 / 12.8 (strips 21.6 / 12.5); 5120 -> 17408 at
+//    four rows, six uneven waves of four groups 42.1 / 40.9, five of two 35.9 / 34.2 (strips 58.8 /
+//    30.1: repacked codes pay 14% there). One projection whose waves take three rounds: four where they
+//    leave five workgroups for eight CUs (11008 -> 3584 at two rows 12.7 / 12.5 -> 9.9 / 9.4).
 //  * 8-bit codes, one or two rows, K up to 8192: the GEMV of four-column groups, one or two passes
-//    over K, groups dealt out XCD by XCD (5120 -> 17408 at one row 47.2 -> 17.6 and 28.7 -> 25.2 us;
-//    together 0.69 at one row, 0.79 at two).
-//  * 8-bit codes in groups of 64 or more, other rows, N of 2048 or more: column blocks of about 32
-//    columns, one or two per CU, K in four splits beyond 96 steps (5120 -> 17408 at 16 rows 52.3 ->
-//    35.8 and 33.7 -> 26.4 us; 14336 -> 4096 at 8 rows 37.8 -> 21.0 and 25.1 -> 16.4 us). Fewer
-//    columns leave CUs idle (8960 -> 1536 at 16 rows 10.3 -> 10.9 us).
+//    over K, groups dealt out XCD by XCD (5120 -> 17408 at one row 48.3 / 28.6 -> 18.1 / 26.2). At two
+//    rows repacked codes pay up to 15% for what MLX rows gain (2048 -> 8192 gate and up 14.8 / 11.3 ->
+//    11.6 / 12.9).
+//  * 8-bit codes in groups of 64 or more, other rows, K up to 96 steps: column blocks over all of K. A
+//    block's waves share K, so short K (up to 24 steps) is fine from 2048 columns on (one projection, 8
+//    rows: 1536 -> 4096 8.6 / 6.6 -> 7.5 / 7.0), longer K only where blocks fill the CUs: from 4608
+//    columns, one projection of more than 16 rows from 6144 (4096 -> 4096 at 16 rows 13.2 / 10.9 -> 15.7
+//    / 12.2 and 5120 -> 2048 11 / 9 -> 18 / 13 would be the loss; 5120 -> 6144 at 16 rows 29 / 21 -> 20 /
+//    16 is the gain). Blocks of about 32 columns, one or two per CU, eight waves up to 16 rows, for two
+//    projections two per CU of four waves (896 -> 4864 at 4 rows 8.3 / 6.3 -> 6.6 / 6.3, 5120 -> 17408
+//    103 / 54 -> 62 / 43). Two corners stay with the strips: 2048 -> 5632 .. 8192 at 8 rows (8.3 / 6.6
+//    against 7.8 / 7.2) and short K beyond 9216 columns at more than 16 rows.
+//  * The same, K beyond 96 steps: four K splits from 3072 columns on (14336 -> 4096 at 8 rows 38.1 / 25.8
+//    -> 22.1 / 17.1), and at 2048 columns, one block per CU, from 17 rows (8192 -> 2048 at 32 rows 14.9 /
+//    12.6 -> 12.8 / 12.0; at 8 rows it would be 10.5 / 9.4 -> 10.8 / 10.4, and 8192 -> 2560 at 32 rows 15.2
+//    / 13.1 -> 18.5 / 16.6).
 bool preferred_qmv(int rows, int K, int N, int nproj, int group_size, int bits, mt_qmv_plan* out) {
   const int cus = device_cus();
   mt_qmv_plan q{};
@@ -444,13 +462,24 @@ bool preferred_qmv(int rows, int K, int N, int nproj, int group_size, int bits, 
   if (bits == 4) {
     const int rounds = (K + 511) / 512;
     if (rows > 4 || rounds > 24 || (rows > 2 && rounds < 8)) return false;
+    if (rows > 2 && rounds > 16 && N >= 20 * cus && N < 24 * cus) return false;
     int per_wave = 1;
     while ((rounds + per_wave - 1) / per_wave > mt::kGemv4MaxWaves) ++per_wave;
     q.kernel = MT_QMV_GEMV4;
     q.tiles = (rounds + per_wave - 1) / per_wave;
-    const int least = rows > 2 ? cus * 3 / 4 : nproj == 1 ? 2 * cus : 2 * cus + cus / 3;
+    const bool shared = nproj == 2 && per_wave > 1 && N >= 16 * cus;
+    for (int waves = mt::kGemv4MaxWaves; shared && waves * 3 >= rounds; --waves)
+      if (rounds % waves == 0) {
+        q.tiles = waves;
+        break;
+      }
+    const bool two = nproj == 2 && ((rows <= 2 && q.tiles < 7) || (shared && q.tiles < 8));
+    const int most = two ? 2 : 4;  // column groups
+    const int few = cus * 5 / 8;
+    const bool long_k = nproj == 1 && per_wave > 2 && N >= 16 * few && N <= 16 * cus;
+    const int least = rows > 2 || long_k ? few : nproj == 1 ? 2 * cus : 2 * cus + cus / 3;
     for (int groups : {4, 2, 1}) {
-      if (N % (4 * groups)) continue;
+      if (groups > most || N % (4 * groups)) continue;
       q.strips = N / (4 * groups);
       if (q.strips >= least &&
           qmv_plan_problem(row_bucket(rows), K, N, nproj, group_size, bits, q).empty())
@@ -473,12 +502,30 @@ bool preferred_qmv(int rows, int K, int N, int nproj, int group_size, int bits, 
       if (qmv_plan_problem(row_bucket(rows), K, N, nproj, group_size, bits, q).empty()) break;
     }
   } else if (group_size >= 64 && N >= 2048) {
+    const bool short_k = K <= 24 * 64;
     q.kernel = MT_QMV_BLOCK;
-    q.ksplit = K / 64 <= 96 ? 1 : 4;
+    q.ksplit = K <= 96 * 64 ? 1 : 4;
     q.strips = N / 32;
-    if (q.ksplit == 1 && q.strips > cus)
-      q.strips = nproj == 1 && N <= 36 * cus ? cus : N <= 36 * 2 * cus ? 2 * cus : q.strips;
-    q.tiles = q.ksplit == 4 ? 4 : rows > 16 ? 4 : nproj == 1 ? 8 : 6;
+    q.tiles = 4;
+    if (q.ksplit == 4) {
+      if (N < 3072 && K <= 128 * 64 && (rows <= 16 || 4 * q.strips > cus)) return false;
+      if (N < 3072 && K <= 176 * 64 && rows > 16 && 4 * q.strips > cus) return false;
+    } else if (rows <= 16) {
+      if (!short_k && N < 18 * cus) return false;
+      if (nproj == 1 && rows <= 8 && !short_k && K <= 36 * 64 && N > 20 * cus && N <= 32 * cus)
+        return false;
+      if (nproj == 2 && N >= 18 * cus && N <= 40 * 2 * cus &&
+          (rows <= 8 || N < 30 * cus || N > 32 * cus))
+        q.strips = 2 * cus;
+      else if (q.strips > cus)
+        q.strips = N <= 36 * cus ? cus : N <= 36 * 2 * cus ? 2 * cus : q.strips;
+      if (q.strips < 2 * cus || nproj == 1) q.tiles = nproj == 1 ? 8 : 6;
+    } else {
+      if (!short_k && N < (nproj == 1 && K > 56 * 64 ? 24 : 18) * cus) return false;
+      if (nproj == 1 && short_k && N > 36 * cus) return false;
+      if (q.strips > cus)
+        q.strips = nproj == 1 && N <= 36 * cus ? cus : N <= 36 * 2 * cus ? 2 * cus : q.strips;
+    }
   } else {
     return false;
   }

@@ -36,6 +36,27 @@ CASES = [
     (128, 9216, 8, 64, "bf16", 1, (4, 20)),              # strips as many as CUs
     (128, 9248, 8, 64, "f16", 1, (4, 20)),               # twice as many
     (128, 18464, 8, 64, "bf16", 2, (3,)),                # one a 32-column strip
+    (4608, 160, 4, 64, "bf16", 2, (1, 2, 4)),            # nine rounds, three waves of three
+    (5120, 3072, 4, 64, "f16", 2, (1, 3, 4)),            # ten, five of two; two column groups
+    (5632, 96, 4, 64, "bf16", 2, (2,)),                  # eleven: uneven waves
+    (8192, 3104, 4, 128, "bf16", 2, (1, 4)),             # sixteen, eight waves: four groups
+    (1536, 9600, 4, 64, "bf16", 2, (1, 2)),              # 600 workgroups of four groups: two all the same
+    (8256, 2528, 4, 64, "f16", 1, (2, 3)),               # 17 rounds, columns beside five for eight CUs
+    (8256, 2560, 4, 64, "bf16", 1, (2, 4)),
+    (8256, 5088, 4, 64, "f16", 1, (3,)),                 # the most columns of three rounds a wave
+    (8256, 5120, 4, 64, "bf16", 1, (2, 4)),
+    (6208, 3040, 8, 64, "bf16", 1, (5, 8)),              # K split, columns below its line
+    (6208, 3072, 8, 64, "f16", 1, (5, 17)),              # and at it
+    (1536, 2048, 8, 64, "f16", 2, (3, 17)),              # short K: from 2048 columns
+    (1600, 4576, 8, 64, "bf16", 1, (3, 8)),              # longer: columns beside 18 per CU
+    (1600, 4608, 8, 64, "f16", 1, (3, 8, 16)),
+    (1600, 4608, 8, 64, "bf16", 2, (3, 17)),
+    (1600, 6112, 8, 64, "f16", 1, (16,)),                # and 24 with more than 16 rows
+    (1600, 6144, 8, 64, "bf16", 1, (8, 17)),
+    (192, 4576, 8, 64, "f16", 2, (4, 32)),               # two projections below two blocks per CU
+    (192, 4608, 8, 64, "bf16", 2, (3, 16)),              # and at them: nine columns a block
+    (128, 20480, 8, 64, "f16", 2, (5,)),                 # forty
+    (128, 20512, 8, 64, "bf16", 2, (5,)),
 ]
 
 
