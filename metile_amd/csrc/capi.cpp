@@ -420,7 +420,7 @@ std::string qmv_plan_problem(int rows, int K, int N, int nproj, int group_size, 
 
 // Where another kernel than the strip kernels above is the better one over both code layouts together
 // (a plan serves both, so that their results stay bit-identical), its plan; else false. Measured over
-// twenty (K, N) from 896 x 4864 to 17408 x 5120, weights from memory, us as (MLX rows, repacked):
+// K 896 to 17408 and N 896 to 18944 (some 400 shapes), weights from memory, us as (MLX rows, repacked):
 //  * 4-bit codes, one or two rows, K up to 12288 (24 rounds of 512, at most three a wave): the
 //    4x4x4-MFMA GEMV with as many waves as rounds allow and the widest column groups that leave about
 //    two workgroups per CU. Both layouts together take 0.75 / 0.78 of the time with one projection
@@ -440,16 +440,16 @@ std::string qmv_plan_problem(int rows, int K, int N, int nproj, int group_size, 
 //    leave five workgroups for eight CUs (11008 -> 3584 at two rows 12.7 / 12.5 -> 9.9 / 9.4).
 //  * 8-bit codes, one or two rows, K up to 8192: the GEMV of four-column groups, one or two passes
 //    over K, groups dealt out XCD by XCD (5120 -> 17408 at one row 48.3 / 28.6 -> 18.1 / 26.2). At two
-//    rows repacked codes pay up to 15% for what MLX rows gain (2048 -> 8192 gate and up 14.8 / 11.3 ->
-//    11.6 / 12.9).
+//    rows, and at one with two projections, repacked codes pay for what MLX rows gain (the worst: 3584 ->
+//    8192 gate and up at two rows 25.1 / 15.8 -> 15.2 / 20.6; both together still take 0.73).
 //  * 8-bit codes in groups of 64 or more, other rows, K up to 96 steps: column blocks over all of K. A
 //    block's waves share K, so short K (up to 24 steps) is fine from 2048 columns on (one projection, 8
-//    rows: 1536 -> 4096 8.6 / 6.6 -> 7.5 / 7.0), longer K only where blocks fill the CUs: from 4608
-//    columns, one projection of more than 16 rows from 6144 (4096 -> 4096 at 16 rows 13.2 / 10.9 -> 15.7
-//    / 12.2 and 5120 -> 2048 11 / 9 -> 18 / 13 would be the loss; 5120 -> 6144 at 16 rows 29 / 21 -> 20 /
-//    16 is the gain). Blocks of about 32 columns, one or two per CU, eight waves up to 16 rows, for two
-//    projections two per CU of four waves (896 -> 4864 at 4 rows 8.3 / 6.3 -> 6.6 / 6.3, 5120 -> 17408
-//    103 / 54 -> 62 / 43). Two corners stay with the strips: 2048 -> 5632 .. 8192 at 8 rows (8.3 / 6.6
+//    rows: 1536 -> 4096 7.1 / 5.3 -> 6.2 / 5.5), longer K only where blocks fill the CUs: from 4608
+//    columns, one projection of more than 16 rows and 56 steps from 6144 (5120 -> 6144 at 16 rows 24.6 /
+//    16.8 -> 17.3 / 13.0; 4096 -> 4096 at 16 rows would be 10.8 / 9.3 -> 12.9 / 10.4, 5120 -> 2048 9.7 / 8.3
+//    -> 15.8 / 11.9). Blocks of about 32 columns, one or two per CU, eight waves up to 16 rows, for two
+//    projections two per CU of four waves (896 -> 4864 at 4 rows 8.3 / 6.3 -> 6.7 / 6.3, 2048 -> 8192 14.9
+//    / 11.4 -> 12.4 / 11.1), one of six where 9 to 16 rows find a 32-column block for nearly every CU. Two corners stay with the strips: 2048 -> 5632 .. 8192 at 8 rows (8.3 / 6.6
 //    against 7.8 / 7.2) and short K beyond 9216 columns at more than 16 rows.
 //  * The same, K beyond 96 steps: four K splits from 3072 columns on (14336 -> 4096 at 8 rows 38.1 / 25.8
 //    -> 22.1 / 17.1), and at 2048 columns, one block per CU, from 17 rows (8192 -> 2048 at 32 rows 14.9 /
@@ -994,8 +994,8 @@ constexpr int kDenseSubChunk = 64;
 // 128 rows 24.5 against 26.3, 8960 -> 3072 37.1 against 40.4 (at 65 rows 31.2 against 29.0). Not gate and
 // up 896 -> 4864 (152 strips) at 100 rows 14.1 against 10.9, 2048 -> 5632 22.8 against 19.4, 1536 -> 8960
 // 27.1 against 25.7; 8192 -> 2048 (256 workgroups) 18.7 against 17.4, 5120 -> 6144 (384) 36.8 against
-// 33.6. With the weights in the caches two chunks are the faster ones by up to 15% in most of these, which
-// a model of many layers does not see.
+// 33.6. With the weights in the caches two chunks are the faster ones in most of these, by up to a quarter,
+// which a model of many layers does not see.
 int dense_row_chunk(int rows, int K, int N, int nproj, int ksplit) {
   if (rows <= kDenseSubChunk) return 0;
   const int cus = device_cus(), wgs = N / 32 * ksplit;
@@ -1268,9 +1268,9 @@ GemmPlan planner_gemm(int M, int K, int N) {
 // fills the CUs (512 x 8960 -> 1536 33.9 against 38.4 us, 128 x 3584 -> 6144 20.7 against 24.8). Its time
 // is a fit (rms error 5%) to 391 measured calls of at most one workgroup a CU, the wide kernel's
 // wide_cost, which is 4 to 8% low. Over 785 calls (33 to 2048 rows, K 896 to 18944, N 896 to 18944,
-// groups of 64) it takes 45, which the wide kernel would run 1.057 times as long (worst 1.20, and 0.97
+// groups of 64) it takes 44, which the wide kernel would run 1.057 times as long (worst 1.20, and 0.97
 // where it is wrong); of the others, none has the ring faster by more than 8%, and most are the wide
-// kernel's by far (geometric mean 0.70).
+// kernel's by far (geometric mean 0.72).
 bool ring_wins(const GemmPlan& g, int M, int K, int N, int group_size, int bits) {
   WidePlan w;
   const int cus = device_cus(), wgs = g.tiles * g.ksplit;
