@@ -449,8 +449,9 @@ std::string qmv_plan_problem(int rows, int K, int N, int nproj, int group_size, 
 //    16.8 -> 17.3 / 13.0; 4096 -> 4096 at 16 rows would be 10.8 / 9.3 -> 12.9 / 10.4, 5120 -> 2048 9.7 / 8.3
 //    -> 15.8 / 11.9). Blocks of about 32 columns, one or two per CU, eight waves up to 16 rows, for two
 //    projections two per CU of four waves (896 -> 4864 at 4 rows 8.3 / 6.3 -> 6.7 / 6.3, 2048 -> 8192 14.9
-//    / 11.4 -> 12.4 / 11.1), one of six where 9 to 16 rows find a 32-column block for nearly every CU. Two corners stay with the strips: 2048 -> 5632 .. 8192 at 8 rows (8.3 / 6.6
-//    against 7.8 / 7.2) and short K beyond 9216 columns at more than 16 rows.
+//    / 11.4 -> 12.4 / 11.1), one of six where 9 to 16 rows find a 32-column block for nearly every CU.
+//    Two corners stay with the strips: 2048 -> 5632 .. 8192 at 8 rows (8.3 / 6.6 against 7.8 / 7.2) and
+//    short K beyond 9216 columns at more than 16 rows.
 //  * The same, K beyond 96 steps: four K splits from 3072 columns on (14336 -> 4096 at 8 rows 38.1 / 25.8
 //    -> 22.1 / 17.1), and at 2048 columns, one block per CU, from 17 rows (8192 -> 2048 at 32 rows 14.9 /
 //    12.6 -> 12.8 / 12.0; at 8 rows it would be 10.5 / 9.4 -> 10.8 / 10.4, and 8192 -> 2560 at 32 rows 15.2
@@ -987,22 +988,22 @@ constexpr int kDenseRowChunk = 128;  // rows per dense dispatch
 constexpr int kDenseSubChunk = 64;
 
 // Rows per chunk of a dispatch, 0 for one chunk. One chunk has the weights delivered once, two bring
-// them to twice as many CUs from one L2: chunked where both chunks fit side by side, a workgroup a CU,
-// and, from 81 rows with K split, where one chunk would leave a short second round of workgroups. Us with
-// weights from memory, two chunks against one, one projection unless said: gate and up 1024 -> 4096 (128
-// strips) at 100 rows 9.9 against 11.7, 4864 -> 896 10.5 against 11.9; 4864 -> 3072 (288 workgroups) at
-// 128 rows 24.5 against 26.3, 8960 -> 3072 37.1 against 40.4 (at 65 rows 31.2 against 29.0). Not gate and
-// up 896 -> 4864 (152 strips) at 100 rows 14.1 against 10.9, 2048 -> 5632 22.8 against 19.4, 1536 -> 8960
-// 27.1 against 25.7; 8192 -> 2048 (256 workgroups) 18.7 against 17.4, 5120 -> 6144 (384) 36.8 against
-// 33.6. With the weights in the caches two chunks are the faster ones in most of these, by up to a quarter,
-// which a model of many layers does not see.
+// them to twice as many CUs from one L2. Two where both fit side by side, a workgroup a CU (us with the
+// weights from memory, two chunks against one: gate and up 1024 -> 4096, 128 strips, at 100 rows 9.9
+// against 11.7; 4864 -> 896 10.5 against 11.9). Beyond that two chunks are the better ones with the
+// weights in the caches and one mostly with weights from memory. Two projections take two where one would
+// leave a short second round of workgroups (1536 -> 8960, 280 strips, at 100 rows 23.1 against 25.2 in the
+// caches, 27.1 against 25.7 from memory; not 896 -> 4864, 152 strips, 10.9 against 11.0 and 14.1 against
+// 10.9). One projection takes two up to 64 MiB of weights and 1.4 workgroups a CU (8192 -> 2048 at 100 rows
+// 14.9 against 16.7 and 18.7 against 17.4; not 5120 -> 6144, 384 workgroups, 29.1 against 32.7 and 36.8
+// against 33.6), and not for K up to 2560 (2560 -> 4096 at 128 rows 13.6 against 12.9 and 18.6 against 14.3).
 int dense_row_chunk(int rows, int K, int N, int nproj, int ksplit) {
   if (rows <= kDenseSubChunk) return 0;
   const int cus = device_cus(), wgs = N / 32 * ksplit;
-  if (2 * wgs <= cus) return kDenseSubChunk;
-  const bool tail = ksplit > 1 && K / 64 > 20 * ksplit && wgs > cus && 3 * wgs <= 4 * cus &&
-                    (size_t)nproj * K * N * 2 <= (96u << 20);
-  return tail && rows > 80 ? kDenseSubChunk : 0;
+  const bool fit = 2 * wgs <= cus;
+  const bool more = nproj == 2 ? wgs > cus && 4 * wgs <= 5 * cus
+                               : K > 2560 && 10 * wgs <= 14 * cus && (size_t)K * N * 2 <= (64u << 20);
+  return fit || more ? kDenseSubChunk : 0;
 }
 
 // Dense plans: the K split of every dispatch of a (K, N) shape. Keyed without the rows, so that
