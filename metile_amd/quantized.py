@@ -155,10 +155,12 @@ def _many_rows_workspace(device, need, least, stream=None):
     return workspace(device, need, stream) if need else None
 
 
-def _qmv_workspace(L, device, m, k, n, group_size, bits, nproj):
-    """The workspace of a QMV or SwiGLU call: with more rows than one dispatch takes, what the wide
-    kernel needs."""
-    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, nproj)
+_FEW_ROWS = 16  # rows that one dispatch takes, whatever the group size
+
+
+def _rows_workspace(L, device, need, m, k, n, group_size, bits, nproj):
+    """The workspace of a QMV or SwiGLU call of more than ``_FEW_ROWS`` rows, ``need`` being what its
+    dispatches take: with more rows than one dispatch takes, what the wide kernel needs."""
     if m <= _dispatch_rows(group_size):
         return workspace(device, need) if need else None
     wide = L.mt_affine_rows_workspace_bytes(m, k, n, group_size, bits, nproj)
@@ -194,7 +196,11 @@ def affine_qmv(values, weight, scales, biases, *, group_size=64, bits=4, residua
     s = scales.contiguous()
     b = biases.contiguous()
     L = _lib.lib()
-    ws = _qmv_workspace(L, values.device, m, k, n, group_size, bits, 1)
+    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, 1)
+    if m > _FEW_ROWS:
+        ws = _rows_workspace(L, values.device, need, m, k, n, group_size, bits, 1)
+    else:
+        ws = workspace(values.device, need) if need else None
     fn = L.mt_affine_qmv_repacked if _repacked(w) else L.mt_affine_qmv
     _lib.check(fn(
         x.data_ptr(), w.data_ptr(), s.data_ptr(), b.data_ptr(), _ptr(res), out.data_ptr(),
@@ -229,7 +235,11 @@ def affine_swiglu(values, gate_weight, gate_scales, gate_biases, up_weight, up_s
     gs, gb = gate_scales.contiguous(), gate_biases.contiguous()
     us, ub = up_scales.contiguous(), up_biases.contiguous()
     L = _lib.lib()
-    ws = _qmv_workspace(L, values.device, m, k, n, group_size, bits, 2)
+    need = L.mt_affine_qmv_workspace_bytes(m, k, n, group_size, bits, 2)
+    if m > _FEW_ROWS:
+        ws = _rows_workspace(L, values.device, need, m, k, n, group_size, bits, 2)
+    else:
+        ws = workspace(values.device, need) if need else None
     fn = L.mt_affine_swiglu_repacked if _repacked(gw) else L.mt_affine_swiglu
     _lib.check(fn(
         x.data_ptr(), gw.data_ptr(), gs.data_ptr(), gb.data_ptr(), uw.data_ptr(), us.data_ptr(),
@@ -288,9 +298,11 @@ def affine_mlp(values, gate, up, down, *, group_size=64, bits=4, residual=None):
     tensors = [_as_u32(gw), gs.contiguous(), gb.contiguous(), _as_u32(uw), us.contiguous(),
                ub.contiguous(), _as_u32(dw), ds.contiguous(), db.contiguous()]
     L = _lib.lib()
-    ws = _mlp_workspace(
-        L, values.device, L.mt_affine_mlp_rows_workspace_bytes(m, hdim, idim, group_size, bits),
-        m, hdim, idim, group_size, bits)
+    need = L.mt_affine_mlp_rows_workspace_bytes(m, hdim, idim, group_size, bits)
+    if m > _FEW_ROWS:
+        ws = _mlp_workspace(L, values.device, need, m, hdim, idim, group_size, bits)
+    else:
+        ws = workspace(values.device, need)
     args = (x.data_ptr(), *[t.data_ptr() for t in tensors], _ptr(res), out.data_ptr(), m, hdim,
             idim, group_size, bits, code)
     tail = (ws.data_ptr(), ws.numel(), _stream_handle(values.device))
@@ -372,8 +384,11 @@ class BoundMlp:
             if need is None:  # installed plans may change the need: refreshed on a refusal
                 need = self.need[m] = L.mt_affine_mlp_rows_workspace_bytes(
                     m, self.hdim, self.idim, self.group_size, self.bits)
-            ws = _mlp_workspace(L, self.device, need, m, self.hdim, self.idim, self.group_size,
-                                self.bits, stream)
+            if m > _FEW_ROWS:
+                ws = _mlp_workspace(L, self.device, need, m, self.hdim, self.idim, self.group_size,
+                                    self.bits, stream)
+            else:
+                ws = workspace(self.device, need, stream)
             st = L.mt_affine_mlp_layouts(
                 x.data_ptr(), *self.wptrs, rptr, out.data_ptr(), m, self.hdim, self.idim,
                 self.group_size, self.bits, self.code, *self.layouts, ws.data_ptr(), ws.numel(),
