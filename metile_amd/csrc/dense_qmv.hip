@@ -51,10 +51,11 @@ __device__ __forceinline__ uint16_t typed_swiglu(float g, float u) {
 
 // Activation tiles above 8 rows go through LDS (XLDS): lane j of an MFMA operand needs row
 // j, so loading the operand directly touches 32 rows (32 cache lines, 32 bytes of each) per
-// instruction; loaded 8 lanes per row instead, every instruction reads 8 whole 128-byte lines. Each wave stages its own tile of the step (wave-private, no barrier) and reads it back
-// in the MFMA layout; the 16-byte chunk c of staged row r sits at slot c ^ (r % 8), so that the
-// eight lanes of a read phase (rows r..r+7, one chunk) hit distinct banks. The operands, and so
-// every MFMA and sum, are the same as with direct loads.
+// instruction; loaded 8 lanes per row instead, every instruction reads 8 whole 128-byte lines.
+// Each wave stages its own tile of the step (wave-private, no barrier) and reads it back in the
+// MFMA layout; the 16-byte chunk c of staged row r sits at slot c ^ (r % 8), so that the eight
+// lanes of a read phase (rows r..r+7, one chunk) hit distinct banks. The operands, and so every
+// MFMA and sum, are the same as with direct loads.
 
 // LDS of one workgroup, 16-byte units: during the K loop each wave's staged activation tile
 // (XLDS) and weight tile ([NPROJ][32 columns][8 chunks], the same swizzle); after it the

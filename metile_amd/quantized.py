@@ -54,8 +54,8 @@ def workspace(device: torch.device, nbytes: int, stream: int | None = None) -> t
     """Return a zero-initialised uint8 workspace of at least ``nbytes`` for the current stream.
 
     Calls on one stream are ordered, so they may share it; the kernels leave its counter
-    region zeroed after each call. ``stream``: the current stream's handle, if the caller has it. A buffer that is outgrown is kept, not freed, so that graphs
-    captured over it stay valid.
+    region zeroed after each call. ``stream``: the current stream's handle, if the caller has
+    it. A buffer that is outgrown is kept, not freed, so that graphs captured over it stay valid.
 
     A buffer is never created or grown during graph capture: its zero fill would only be
     recorded into that graph, not run, and a later call or graph on the stream would find it
@@ -447,10 +447,11 @@ def affine_repack(weight, *, bits=4):
 
 
 def affine_matmul(values, weight, scales, biases, *, group_size=64, bits=4):
-    """Prefill ``values @ dequantize(weight).T`` for many rows: codes are dequantized to the
-    activation type in LDS and multiplied on the matrix cores (fp32 accumulation), the
-    semantics of MLX's quantized matmul for large row counts
-    (``metile/backends/mlx_affine.py:142-154``)."""
+    """Prefill ``values @ dequantize(weight).T`` for many rows on the matrix cores (fp32
+    accumulation), the semantics of MLX's quantized matmul for large row counts
+    (``metile/backends/mlx_affine.py:142-154``). Calls that reach the wide kernel multiply the
+    codes themselves as whole numbers and apply scale and bias to fp32 group sums; the ring GEMM
+    (4 bits, where it is the faster one) dequantizes to the activation type in LDS."""
     if biases is None:
         raise ValueError("affine matmul requires affine quantization biases")
     _require_device(values, weight, scales, biases)
@@ -799,8 +800,9 @@ def mlx_affine_matmul_dispatches():
 def mlx_affine_matmul(values, weight, *, autotune=True):
     """Drop-in for ``mlx_affine_matmul`` (``metile/backends/mlx_affine.py:359-406``) with the
     reference's guards; with ``autotune`` the first call of a shape takes its tuned GEMM plan
-    (``metile_amd.tuning``), as the reference's tuned dispatch does (``:380-406``). The reference's Metal path takes float16 only; the gfx950 GEMM also
-    takes bfloat16 (BASELINE config 4 is bf16), and any other dtype raises ``TypeError``."""
+    (``metile_amd.tuning``), as the reference's tuned dispatch does (``:380-406``). The
+    reference's Metal path takes float16 only; the gfx950 GEMM also takes bfloat16, and any other
+    dtype raises ``TypeError``."""
     if not isinstance(weight, AffineWeight):
         raise TypeError("weight must be an AffineWeight")
     if values.ndim < 2 or values.shape[-1] != weight.shape[0]:

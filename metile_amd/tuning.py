@@ -1,7 +1,7 @@
 """Plan tuning with a persistent decision cache.
 
 Every C-ABI call plans itself from its shape (split-K, column strips, kernel). The planner's rules
-were measured at the BASELINE shapes; for any other shape this module measures the plans the
+were measured over a range of shapes; for a shape of its own this module measures the plans the
 library lists for it (``mt_affine_qmv_plan_candidates``, ``mt_affine_gemm_plan_candidates``) and
 installs the fastest (``mt_affine_*_plan_set``), so that later calls of that shape take it. The
 decision is appended to a persistent log keyed by everything that can change it, the role the

@@ -1,7 +1,7 @@
 """Calls of more rows than one small-row dispatch takes, through the entry points: the wide kernel's
 tile edges (rows and columns beside multiples of 32, 64, 96 and 128), one K step and step counts
 beside its four- and eight-step loop and its 16-group chunks, odd group counts (scale rows that start
-inside a dword), K splits, both code widths, all group sizes, both types, both layouts, residuals and
+inside a dword), K splits, both code widths, groups of 32 to 4096, both types, both layouts, residuals and
 the SwiGLU epilogue, against the oracle.
 
 The bars are the contract's: 2e-3 of the largest output after removing the final rounding, and at
@@ -41,6 +41,11 @@ CASES = [
     (100, 1152, 96, 8, 128, "f16", 1, True, False),
     (130, 2048, 288, 8, 32, "bf16", 1, True, True),
     (36, 5120, 64, 8, 64, "f16", 1, False, True),       # K splits
+    (300, 2048, 544, 4, 64, "f16", 1, True, False),     # the same over ten row dispatches
+    (17, 2560, 64, 8, 32, "f16", 1, False, True),
+    (64, 8192, 64, 4, 512, "bf16", 1, True, True),      # groups beyond four steps: splits of whole ones
+    (40, 8192, 96, 8, 1024, "f16", 2, False, False),
+    (100, 4096, 96, 4, 4096, "bf16", 1, False, False),  # one group a row
 ]
 
 
@@ -85,21 +90,38 @@ def test_wide_meets_the_contract(m, k, n, bits, g, dtype, nproj, residual, repac
     same = np.mean(O.to_f32(y, dtype) == rounded)
     print(f"[wide] tolerance_error={err:.2e} exact={same:.5f}", flush=True)
     assert err <= TOL and same >= (0.98 if dtype == "bf16" else 0.90)
-    # with the sizes of the row dispatches the call runs as before (the same contract)
+    # With the workspace of the row dispatches the call runs as them (where the wide kernel needs no
+    # more, it runs all the same): the bits of the slices.
     lib = _lib.lib()
     need = lib.mt_affine_qmv_workspace_bytes(m, k, n, g, bits, nproj)
     ws = torch.zeros(max(need, 1), dtype=torch.uint8, device="cuda")
     out = torch.empty_like(got)
     args = [xt.data_ptr(), *(t.data_ptr() for triple in triples for t in triple)]
     if nproj == 1:
-        args.append(act_to_torch(res, dtype).data_ptr() if residual else None)
-    keep = act_to_torch(res, dtype) if residual else None
-    if residual:
-        args[-1] = keep.data_ptr()
+        args.append(rt.data_ptr() if residual else None)
     _lib.check(_fn(nproj, repacked)(
         *args, out.data_ptr(), m, k, n, g, bits, _lib.MT_BF16 if dtype == "bf16" else _lib.MT_F16,
         ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream))
     assert O.tolerance_error(torch_to_act(out, dtype), ref, dtype) <= TOL
+    if lib.mt_affine_rows_workspace_bytes(m, k, n, g, bits, nproj) <= need:
+        return
+    chunk = 16 if g == 32 else 32
+    for i in range(0, m, chunk):
+        part = xt[i:i + chunk]
+        alone = (mt.affine_swiglu(part, *triples[0], *triples[1], group_size=g, bits=bits)
+                 if nproj == 2 else
+                 mt.affine_qmv(part, *triples[0], group_size=g, bits=bits,
+                               residual=rt[i:i + chunk] if residual else None))
+        assert torch.equal(out[i:i + chunk].view(torch.int16), alone.view(torch.int16))
+
+
+def test_cases_cover_row_dispatches_in_place_of_the_wide_kernel():
+    """Some cases' second half runs row dispatches: several chunks, groups of 32, both projections."""
+    lib = _lib.lib()
+    split = [c for c in CASES if lib.mt_affine_rows_workspace_bytes(c[0], c[1], c[2], c[4], c[3], c[6])
+             > lib.mt_affine_qmv_workspace_bytes(c[0], c[1], c[2], c[4], c[3], c[6])]
+    assert any(c[0] > 64 for c in split) and {c[3] for c in split} == {4, 8}
+    assert {c[6] for c in split if c[4] == 32} == {1, 2} and any(c[4] > 256 for c in split)
 
 
 @pytest.mark.gpu
