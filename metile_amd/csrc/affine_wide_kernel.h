@@ -27,14 +27,20 @@
 // and the next step's first operands are read, whose latency that row tile hides. The scales and
 // biases of 16 groups are staged in LDS a chunk ahead.
 //
-// Measured (MI355X, 4-bit groups of 64, best plan; before: the ring GEMM for one projection, 32-row
-// dispatches for the others): 2048 x 14336 x 4096 f16 397 -> 259 us (928 TFLOP/s; torch's dense f16
-// product 231 us), 512 x 1536 x 8960 30.3 -> 25.9 us, SwiGLU 333 x 1536 x 8960 (x 2) about 180 ->
-// 32 us, 48 rows 22.6 -> 15.0 us. At 2048 rows the matrix cores are busy half of the time and the
-// other vector instructions take the other half: 110 per wave and step (64 FMAs, 36 for codes) beside
-// 18 MFMAs. Tried: waves of 64 columns, one a SIMD with 512 registers (348 us: nothing hides a wait);
-// waves of 64 x 64 (317 us, spills); a barrier every second step (267 us); codes through LDS (260 us,
-// the same, and 8 KiB a stage).
+// Measured (MI355X, 4-bit groups of 64, weights from memory; before: the ring GEMM for one projection,
+// 32-row dispatches for the others): 2048 x 14336 x 4096 f16 437 -> 277 us, bf16 404 -> 262 (868 and 918
+// TFLOP/s; torch's dense products 223 and 214 us), 512 x 1536 x 8960 bf16 30.9 -> 27.0 us, SwiGLU
+// 1536 -> 8960 of 333 rows 148 -> 33.4 us over MLX rows and 106 -> 32.2 repacked, of 48 rows 27.2 -> 16.7
+// and 18.5 -> 15.9. At 2048 rows the matrix cores are busy 55% of a SIMD's clocks and vector
+// instructions are issued in 54% (131 per wave and step, 64 FMAs and 36 for codes, beside 20 MFMAs); a
+// wave waits 35% of its life. Tried at that size in f16 (259 us with inputs that
+// let the clocks run higher): waves of 64 columns, one a SIMD with 512 registers (348 us: nothing hides a
+// wait); waves of 64 x 64 (317 us, spills); a barrier every second step (267 us); codes through LDS (260
+// us, the same, and 8 KiB a stage).
+// Groups of 32 keep two chains and two scales a step and spill: 4 to 66 registers, at most 180 bytes a
+// lane, in the 64-row instances and in those of 96 and 128 rows whose registers two waves a SIMD share;
+// 8-bit groups of 64 spill 2 to 5 in three of the 64 x 64 instances. The planner's costs were fitted with
+// that in.
 #pragma once
 
 #include "affine_wide.h"

@@ -302,13 +302,15 @@ __global__ __launch_bounds__(kThreads, 2) void dense_qmv_kernel(const DenseParam
 // The sums are those of the kernel above to the bit: each K quarter of the split is one MFMA chain
 // from zero, in the same operand order, and the quarters are added in order.
 //
-// What bounds it: 2048 -> 8192 runs at the weights' rate from memory, more strips and rows at
-// what a CU receives (about 20 bytes a clock, activations and weights together; a ring of six steps
-// instead of three, or reading operands a step ahead, changed nothing). Measured (MI355X, bf16, weights
-// from memory, gate and up / down, us; before: K quarter a wave, over 64 rows in two chunks): 2048 ->
-// 8192 at 64 rows 18.5 / 14.3 -> 18.3 / 14.0 (at 33 rows 16.6 / 12.6 -> 17.9 / 12.5: the one size where
-// the kernel before was faster), at 128 26.5 / 21.4 -> 21.4 / 20.9; 4096 -> 14336 at 100 rows 102 / 55 ->
-// 70 / 45; 5120 -> 17408 at 100 rows 181 / 88 -> 110 / 78.
+// What bounds it: 2048 -> 8192 runs at the weights' rate from memory; more strips and rows, one
+// workgroup a CU, at what that workgroup receives: about 20 bytes a clock, activations and weights
+// together (a ring of six steps instead of three, or reading operands a step ahead, changed nothing; two
+// workgroups a CU, the down projection's four splits, receive 31). Measured (MI355X, bf16, weights from
+// memory, gate and up / down, us; before: a K quarter a wave, over 64 rows in two chunks): 2048 -> 8192 at
+// 64 rows 18.6 / 14.4 -> 18.3 / 13.9, at 128 26.6 / 21.5 -> 21.6 / 21.8; 4096 -> 14336 at 100 rows 102 /
+// 55 -> 72 / 45; 5120 -> 17408 at 100 rows 181 / 88 -> 113 / 79. The kernel before was the faster one for
+// gate and up of 2048 -> 8192 at 33 rows (17.4 -> 18.9) and of 1536 -> 8960 at 128 (28.5 -> 29.7), and
+// with 178 MB of weights left in the caches (5120 -> 17408, down, 100 rows: 70.9 -> 78.6).
 // NT: weights read once, with the non-temporal hint; not where a second row chunk or a later launch of
 // the call reads them again (5120 -> 17408 at 160 rows, 128 and 32, with the hint 201 / 133, without 186 /
 // 125 us).
